@@ -10,10 +10,8 @@
 // multiplicity) and sums n_b*h_b over the rest.  This file takes the counts as
 // given -- an injected (B,F,R) array, the exact parity path -- and holds the
 // merge shared with the drawn-count kernels of realize_gap.hip:
-//   * a workgroup handles one frequency and one chunk of bins, one thread per
-//     realization; bin data (h, priority key, parameters) are staged through
-//     LDS and shared by all realizations;
-//   * each thread keeps the L best instances of its chunk in registers
+//   * a thread handles one (frequency, realization) column and one chunk of bins;
+//   * it keeps the L best instances of its chunk in registers
 //     (priority = order rank for the sorted walk, (h desc, bin asc) for argmax)
 //     and the FP64 totals sum(n h), sum(n h p_k);
 //   * a merge kernel combines the chunk lists per (f, r); the background is
@@ -29,8 +27,10 @@ namespace hd {
 
 constexpr int LMAX = 16;
 constexpr int NPAR_MAX = 8;
-constexpr int RZ_CHUNK = 16384;   // bins per workgroup
-constexpr int RZ_SUB = 256;       // bins staged in LDS at a time
+constexpr int RZ_THREADS = 256;   // columns (f, r) per workgroup, one per thread
+constexpr int RZ_MIN_CHUNK = 64;  // bins per chunk, at least
+constexpr int RZ_WAVES = 8192;    // waves the chunk count aims at
+constexpr int RZ_MAX_CHUNKS = 512;
 constexpr uint64_t KEY_NONE = ~0ull;
 
 struct RealizeArgs {
@@ -52,128 +52,11 @@ struct RealizeArgs {
 
 constexpr uint32_t KEY32_NONE = 0xffffffffu;
 
-// store / load one slot of a partial list in the mode's layout
-__device__ __forceinline__ void part_store(const RealizeArgs& A, int64_t o, uint64_t k, int32_t b) {
-    if (A.mode == HD_SEL_SORTED) {
-        ((uint32_t*)A.p_key)[o] = (k == KEY_NONE) ? KEY32_NONE : (uint32_t)k;
-    } else {
-        A.p_key[o] = k;
-        A.p_bin[o] = b;
-    }
-}
-
 // ascending image of a double, so that larger h -> smaller key when inverted
 __device__ __forceinline__ uint64_t h_priority(double h) {
     uint64_t u = (uint64_t)__double_as_longlong(h);
     u = (u & 0x8000000000000000ull) ? ~u : (u | 0x8000000000000000ull);
     return ~u;
-}
-
-__device__ __forceinline__ bool better(uint64_t ka, int32_t ba, uint64_t kb, int32_t bb) {
-    return (ka < kb) || (ka == kb && ba < bb);
-}
-
-// insert one instance into a sorted register list of LMAX slots
-__device__ __forceinline__ void list_insert(uint64_t (&lk)[LMAX], int32_t (&lb)[LMAX], uint64_t k, int32_t b) {
-#pragma unroll
-    for (int i = 0; i < LMAX; i++) {
-        bool sw = better(k, b, lk[i], lb[i]);
-        uint64_t tk = lk[i];
-        int32_t tb = lb[i];
-        lk[i] = sw ? k : tk;
-        lb[i] = sw ? b : tb;
-        k = sw ? tk : k;
-        b = sw ? tb : b;
-    }
-}
-
-__global__ void __launch_bounds__(512) k_realize_chunk(RealizeArgs A) {
-    __shared__ double s_h[RZ_SUB];
-    __shared__ uint64_t s_key[RZ_SUB];
-    __shared__ double s_par[NPAR_MAX][RZ_SUB];
-
-    const int f = blockIdx.y;
-    const int chunk = blockIdx.x;
-    const int64_t b0 = (int64_t)chunk * RZ_CHUNK;
-    const int64_t b1 = min(b0 + (int64_t)RZ_CHUNK, A.B);
-    const int F = A.F, R = A.R, L = A.L;
-    const bool use_list = (A.mode != HD_SEL_NONE);
-    const bool sorted_mode = (A.mode == HD_SEL_SORTED);
-    const bool skip_zero_h = (A.flags & HD_FLAG_SKIP_ZERO_H) != 0;
-
-    for (int r0 = 0; r0 < R; r0 += blockDim.x) {
-        const int r = r0 + threadIdx.x;
-        const bool active = r < R;
-        uint64_t lk[LMAX];
-        int32_t lb[LMAX];
-#pragma unroll
-        for (int i = 0; i < LMAX; i++) {
-            lk[i] = KEY_NONE;
-            lb[i] = 0x7fffffff;
-        }
-        double total = 0.0;
-        double ptot[NPAR_MAX];
-#pragma unroll
-        for (int k = 0; k < NPAR_MAX; k++) ptot[k] = 0.0;
-
-        for (int64_t s0 = b0; s0 < b1; s0 += RZ_SUB) {
-            const int ns = (int)min((int64_t)RZ_SUB, b1 - s0);
-            __syncthreads();
-            for (int c = threadIdx.x; c < ns; c += blockDim.x) {
-                int64_t b = s0 + c;
-                double h = A.h2fdf[b * F + f];
-                s_h[c] = h;
-                s_key[c] = sorted_mode ? (uint64_t)A.rank[b] : h_priority(h);
-                for (int k = 0; k < A.npar; k++) s_par[k][c] = A.par[((int64_t)k * A.B + b) * F + f];
-            }
-            __syncthreads();
-            if (!active) continue;
-            for (int c = 0; c < ns; c++) {
-                const int64_t b = s0 + c;
-                const double n = A.counts[(b * F + f) * R + r];
-                const double h = s_h[c];
-                if (sorted_mode) {
-                    if (n < 1) continue;
-                    if (skip_zero_h && h == 0) continue;
-                } else {
-                    if (n == 0) continue;
-                }
-                const double nh = n * h;
-                total += nh;
-                for (int k = 0; k < A.npar; k++) ptot[k] += nh * s_par[k][c];
-                if (use_list && n > 0) {
-                    if (!sorted_mode && !(h > 0)) continue;   // argmax: strict cur > max >= 0
-                    const uint64_t key = s_key[c];
-                    const int32_t bb = (int32_t)b;
-                    // the same (key, bin) for every instance of this bin
-                    int ninst = (int)min(ceil(n), (double)L);
-                    for (int i = 0; i < ninst; i++) {
-                        // compare against slot L-1 (dynamic index avoided: scan)
-                        uint64_t wk = KEY_NONE;
-                        int32_t wb = 0x7fffffff;
-#pragma unroll
-                        for (int j = 0; j < LMAX; j++)
-                            if (j == L - 1) { wk = lk[j]; wb = lb[j]; }
-                        if (!better(key, bb, wk, wb)) break;
-                        list_insert(lk, lb, key, bb);
-                    }
-                }
-            }
-        }
-        if (active) {
-            int64_t pr = ((int64_t)f * A.nchunks + chunk) * R + r;
-            A.p_total[pr] = total;
-            for (int k = 0; k < A.npar; k++) A.p_ptot[(int64_t)k * F * A.nchunks * R + pr] = ptot[k];
-            if (use_list) {
-#pragma unroll
-                for (int j = 0; j < LMAX; j++)
-                    if (j < L) {
-                        const int64_t o = ((pr / R) * L + j) * R + (pr % R);
-                        part_store(A, o, lk[j], lb[j]);
-                    }
-            }
-        }
-    }
 }
 
 // Running list of the merges: LM slots (LM = L for the common L = 1, 5, 10; 16 slots holding
@@ -225,6 +108,96 @@ struct MergeList {
     }
 };
 
+// Chunk partials of given counts.  A thread owns one column (f, r) of the (B, F R) counts and
+// walks its chunk's bins: a wave then reads 512 contiguous bytes per bin, across frequency
+// boundaries too, so ragged R wastes no lanes.  RZ_U bins are loaded ahead of their use.  Bound by
+// the counts' bytes: the chunks are cut so that the launch has about RZ_WAVES waves whatever R is
+// (one frequency per workgroup and chunks of 16384 bins left 160 waves at 120,000 x 20 x 50, every
+// load's latency exposed: 9.94 ms there, 98 GB/s; 0.30 ms and 3.3 TB/s now).
+// LM, S32: the list as in the merges.  NP = 0: no parameters.
+constexpr int RZ_U = 8;
+template <int LM, bool S32, int NP>
+__global__ void __launch_bounds__(RZ_THREADS) k_realize_chunk(RealizeArgs A, int chunk_bins) {
+    using List = MergeList<LM, S32>;
+    using Key = typename List::Key;
+    const int64_t FR = (int64_t)A.F * A.R;
+    const int64_t col = (int64_t)blockIdx.x * RZ_THREADS + threadIdx.x;
+    if (col >= FR) return;
+    const int chunk = blockIdx.y;
+    const int f = (int)(col / A.R), r = (int)(col - (int64_t)f * A.R);
+    const int F = A.F, R = A.R;
+    const int L = (LM == 16) ? A.L : LM;
+    const int64_t b0 = (int64_t)chunk * chunk_bins, b1 = min(b0 + (int64_t)chunk_bins, A.B);
+    const bool use_list = (A.mode != HD_SEL_NONE);
+    const bool skip_zero_h = S32 && (A.flags & HD_FLAG_SKIP_ZERO_H) != 0;
+    List list;
+    list.init();
+    double total = 0.0;
+    double ptot[NP > 0 ? NP : 1];
+#pragma unroll
+    for (int k = 0; k < (NP > 0 ? NP : 1); k++) ptot[k] = 0.0;
+    for (int64_t s = b0; s < b1; s += RZ_U) {
+        double nn[RZ_U], hh[RZ_U];
+        int32_t rk[RZ_U];
+#pragma unroll
+        for (int u = 0; u < RZ_U; u++) {   // every load issued first (the last bin again past the end)
+            const int64_t b = min(s + u, b1 - 1);
+            nn[u] = A.counts[b * FR + col];
+            hh[u] = A.h2fdf[b * F + f];
+            rk[u] = S32 ? A.rank[b] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < RZ_U; u++) {
+            const int64_t b = s + u;
+            const double n = nn[u], h = hh[u];
+            // the sorted walk skips counts below one (and, on request, bins without strain)
+            bool on = b < b1;
+            if (S32) on = on && !(n < 1) && !(skip_zero_h && h == 0);
+            else on = on && (n != 0);
+            if (!on) continue;
+            const double nh = n * h;
+            total += nh;
+            if (NP > 0) {
+#pragma unroll
+                for (int k = 0; k < (NP > 0 ? NP : 1); k++)
+                    if (k < A.npar) ptot[k] += nh * A.par[((int64_t)k * A.B + b) * F + f];
+            }
+            if (use_list && n > 0 && (S32 || h > 0)) {   // argmax: strict cur > max >= 0
+                const Key key = S32 ? (Key)(uint32_t)rk[u] : (Key)h_priority(h);
+                const int32_t bb = (int32_t)b;
+                const int ninst = (int)min(ceil(n), (double)L);   // the same (key, bin) for every instance
+                for (int i = 0; i < ninst; i++) {
+                    Key wk;
+                    int32_t wb;
+                    list.worst(L, wk, wb);
+                    if (!List::better(key, bb, wk, wb)) break;
+                    list.insert(key, bb);
+                }
+            }
+        }
+    }
+    const int64_t pr = ((int64_t)f * A.nchunks + chunk) * R + r;
+    A.p_total[pr] = total;
+    if (NP > 0) {
+#pragma unroll
+        for (int k = 0; k < (NP > 0 ? NP : 1); k++)
+            if (k < A.npar) A.p_ptot[(int64_t)k * F * A.nchunks * R + pr] = ptot[k];
+    }
+    if (use_list) {
+#pragma unroll
+        for (int j = 0; j < LM; j++)
+            if (j < L) {
+                const int64_t o = (((int64_t)f * A.nchunks + chunk) * L + j) * R + r;
+                if (S32) {
+                    ((uint32_t*)A.p_key)[o] = (uint32_t)list.k[j];
+                } else {
+                    A.p_key[o] = (uint64_t)list.k[j];
+                    A.p_bin[o] = list.b[j];
+                }
+            }
+    }
+}
+
 // Merge of chunk partials [c0, c1) of (f, r) into a running list, total and parameter totals.
 template <int LM, bool S32>
 __device__ __forceinline__ void merge_chunks(const RealizeArgs& A, int f, int r, int c0, int c1,
@@ -267,7 +240,15 @@ __device__ __forceinline__ void merge_chunks(const RealizeArgs& A, int f, int r,
     }
 }
 
-constexpr int MERGE_GROUPS = 8;
+// Groups of the first merge stage, of NC chunks: none for few chunks, 8 where (f, group, r) already
+// fills the GPU, else about sqrt(NC), the fewest serial steps over both stages.
+int realize_merge_groups(int F, int R, int NC) {
+    if (NC <= 16) return 0;
+    if ((int64_t)F * R * 8 >= 65536) return 8;
+    int g = 8;
+    while (g < 32 && g * g < NC) g++;
+    return g;
+}
 
 // First merge stage: thread per (f, group, r) merges the group's chunks and writes a partial of
 // the same layout with G "chunks", so that the final merge reads G partials instead of NC (the
@@ -366,14 +347,35 @@ __global__ void k_rank_from_order(const int64_t* __restrict__ order, int64_t B, 
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-size_t realize_group_ws(int F, int R, int L, int npar);
+int realize_merge_groups(int F, int R, int NC);
+size_t realize_group_ws(int F, int R, int L, int npar, int G);
 int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* order, int64_t B, int F, int R, int L,
                          int mode, int npar, int nchunks, const double* p_total, const double* p_ptot, const uint64_t* p_key,
                          const int32_t* p_bin, double* hc2ss, int64_t* ssidx, double* hc2bg, double* bgpar,
-                         void* group_ws, hipStream_t st);
+                         void* group_ws, int G, hipStream_t st);
+
+// Bins per chunk of given counts: about RZ_WAVES waves over the columns, at least RZ_MIN_CHUNK
+// bins (a chunk's partial costs as much as a few bins) and at most RZ_MAX_CHUNKS chunks (the merge
+// walks them).
+static int counts_chunk_bins(int64_t B, int F, int R) {
+    const int64_t waves = cdiv((int64_t)F * R, 64);
+    int64_t nch = cdiv(RZ_WAVES, waves);
+    nch = min(nch, min((int64_t)RZ_MAX_CHUNKS, cdiv(B, RZ_MIN_CHUNK)));
+    return (int)(cdiv(cdiv(B, nch), RZ_U) * RZ_U);
+}
+
+template <int LM, bool S32>
+static int chunk_launch(const RealizeArgs& A, int bins, hipStream_t st) {
+    const dim3 grid((unsigned)cdiv((int64_t)A.F * A.R, RZ_THREADS), (unsigned)A.nchunks);
+    if (A.npar == 0)
+        hipLaunchKernelGGL((k_realize_chunk<LM, S32, 0>), grid, dim3(RZ_THREADS), 0, st, A, bins);
+    else
+        hipLaunchKernelGGL((k_realize_chunk<LM, S32, NPAR_MAX>), grid, dim3(RZ_THREADS), 0, st, A, bins);
+    return check_launch("k_realize_chunk");
+}
 
 static size_t realize_ws(int64_t B, int F, int R, int L, int npar) {
-    int64_t nch = cdiv(B, RZ_CHUNK);
+    int64_t nch = cdiv(B, counts_chunk_bins(B, F, R));
     size_t pr = (size_t)F * nch * R;
     size_t s = 0;
     s += align256((size_t)B * 4);               // rank
@@ -381,7 +383,7 @@ static size_t realize_ws(int64_t B, int F, int R, int L, int npar) {
     s += align256(pr * 8 * (size_t)npar);       // param totals
     s += align256(pr * 8 * (size_t)L);          // keys
     s += align256(pr * 4 * (size_t)L);          // bins
-    s += align256(realize_group_ws(F, R, L, npar));   // first merge stage
+    s += align256(realize_group_ws(F, R, L, npar, realize_merge_groups(F, R, (int)nch)));   // first merge stage
     return s + 256;
 }
 
@@ -415,7 +417,8 @@ static int realize_counts_impl(const double* counts, const double* h2fdf, const 
     A.mode = mode;
     A.flags = flags;
     A.npar = npar;
-    A.nchunks = (int)cdiv(B, RZ_CHUNK);
+    const int bins = counts_chunk_bins(B, F, R);
+    A.nchunks = (int)cdiv(B, bins);
     size_t pr = (size_t)F * A.nchunks * R;
     char* p = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
     int32_t* rank = (int32_t*)p;  p += align256((size_t)B * 4);
@@ -432,29 +435,37 @@ static int realize_counts_impl(const double* counts, const double* h2fdf, const 
         int rc = check_launch("k_rank_from_order");
         if (rc) return rc;
     }
-    int threads = (int)min((int64_t)512, cdiv(R, 64) * 64);
-    dim3 grid(A.nchunks, F);
-    hipLaunchKernelGGL(k_realize_chunk, grid, dim3(threads), 0, st, A);
-    int rc = check_launch("k_realize_chunk");
+    int rc;
+    if (mode == HD_SEL_SORTED) {
+        if (L == 1) rc = chunk_launch<1, true>(A, bins, st);
+        else if (L == 5) rc = chunk_launch<5, true>(A, bins, st);
+        else if (L == 10) rc = chunk_launch<10, true>(A, bins, st);
+        else rc = chunk_launch<16, true>(A, bins, st);
+    } else if (mode == HD_SEL_ARGMAX) {
+        if (L == 1) rc = chunk_launch<1, false>(A, bins, st);
+        else rc = chunk_launch<16, false>(A, bins, st);
+    } else {
+        rc = chunk_launch<1, false>(A, bins, st);   // no lists
+    }
     if (rc) return rc;
-    // the same two-stage merge as the drawn-count kernels (groups of chunks first when there are many)
+    // the same merge as the drawn-count kernels (groups of chunks first when there are many)
     return realize_merge_launch(h2fdf, par, order, B, F, R, L, mode, npar, A.nchunks, A.p_total, A.p_ptot, A.p_key,
-                                A.p_bin, hc2ss, ssidx, hc2bg, (npar > 0) ? bgpar : nullptr, group_ws, st);
+                                A.p_bin, hc2ss, ssidx, hc2bg, (npar > 0) ? bgpar : nullptr, group_ws,
+                                realize_merge_groups(F, R, A.nchunks), st);
 }
 
 // Merge of per-chunk partials, shared with the drawn-count kernel (realize_gap.hip).
-size_t realize_group_ws(int F, int R, int L, int npar) {
-    return (size_t)F * MERGE_GROUPS * R * (sizeof(double) * (1 + (size_t)npar) + (sizeof(uint64_t) + sizeof(int32_t)) * (size_t)L) +
+size_t realize_group_ws(int F, int R, int L, int npar, int G) {
+    return (size_t)F * G * R * (sizeof(double) * (1 + (size_t)npar) + (sizeof(uint64_t) + sizeof(int32_t)) * (size_t)L) +
            4 * 256;
 }
 
 // the two merge stages for list capacity LM and key width (S32: the sorted walk's ranks)
 template <int LM, bool S32>
-static int merge_launch_k(RealizeArgs A, void* group_ws, double* hc2ss, int64_t* ssidx, double* hc2bg, double* bgpar,
+static int merge_launch_k(RealizeArgs A, void* group_ws, int G, double* hc2ss, int64_t* ssidx, double* hc2bg, double* bgpar,
                           hipStream_t st) {
     const int F = A.F, R = A.R, L = A.L, npar = A.npar;
-    if (group_ws && A.nchunks > 2 * MERGE_GROUPS) {
-        const int G = MERGE_GROUPS;
+    if (G > 0) {
         const size_t n = (size_t)F * G * R;
         char* w = (char*)(((uintptr_t)group_ws + 255) & ~(uintptr_t)255);
         double* q_total = (double*)w;         w += n * sizeof(double);
@@ -479,7 +490,7 @@ static int merge_launch_k(RealizeArgs A, void* group_ws, double* hc2ss, int64_t*
 int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* order, int64_t B, int F, int R, int L,
                          int mode, int npar, int nchunks, const double* p_total, const double* p_ptot, const uint64_t* p_key,
                          const int32_t* p_bin, double* hc2ss, int64_t* ssidx, double* hc2bg, double* bgpar,
-                         void* group_ws, hipStream_t st) {
+                         void* group_ws, int G, hipStream_t st) {
     RealizeArgs A;
     A.counts = nullptr;
     A.h2fdf = h2fdf;
@@ -499,18 +510,18 @@ int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* 
     A.p_key = const_cast<uint64_t*>(p_key);
     A.p_bin = const_cast<int32_t*>(p_bin);
     if (mode == HD_SEL_SORTED) {
-        if (L == 1) return merge_launch_k<1, true>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        if (L == 5) return merge_launch_k<5, true>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        if (L == 10) return merge_launch_k<10, true>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        return merge_launch_k<16, true>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 1) return merge_launch_k<1, true>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 5) return merge_launch_k<5, true>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 10) return merge_launch_k<10, true>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        return merge_launch_k<16, true>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
     }
     if (mode == HD_SEL_ARGMAX) {
-        if (L == 1) return merge_launch_k<1, false>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        if (L == 5) return merge_launch_k<5, false>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        if (L == 10) return merge_launch_k<10, false>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
-        return merge_launch_k<16, false>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 1) return merge_launch_k<1, false>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 5) return merge_launch_k<5, false>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        if (L == 10) return merge_launch_k<10, false>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
+        return merge_launch_k<16, false>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);
     }
-    return merge_launch_k<1, false>(A, group_ws, hc2ss, ssidx, hc2bg, bgpar, st);   // no lists
+    return merge_launch_k<1, false>(A, group_ws, G, hc2ss, ssidx, hc2bg, bgpar, st);   // no lists
 }
 
 int rank_from_order_launch(const int64_t* order, int64_t B, int32_t* rank, hipStream_t st) {

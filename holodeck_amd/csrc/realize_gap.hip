@@ -1249,8 +1249,9 @@ __global__ void __launch_bounds__(256) k_table_draw_pair_hook(const uint32_t* ta
 int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* order, int64_t B, int F, int R, int L,
                          int mode, int npar, int nchunks, const double* p_total, const double* p_ptot, const uint64_t* p_key,
                          const int32_t* p_bin, double* hc2ss, int64_t* ssidx, double* hc2bg, double* bgpar,
-                         void* group_ws, hipStream_t st);
-size_t realize_group_ws(int F, int R, int L, int npar);
+                         void* group_ws, int G, hipStream_t st);
+int realize_merge_groups(int F, int R, int NC);
+size_t realize_group_ws(int F, int R, int L, int npar, int G);
 int rank_from_order_launch(const int64_t* order, int64_t B, int32_t* rank, hipStream_t st);
 
 static size_t gz_align(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1290,7 +1291,7 @@ static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
     s += 2 * gz_align(slots * 8 * (size_t)npar);           // params
     s += gz_align(pr * 8) + gz_align(pr * 8 * (size_t)npar) + gz_align(pr * 8 * (size_t)L) +
          gz_align(pr * 4 * (size_t)L);
-    s += gz_align(realize_group_ws(F, R, L, npar));          // first merge stage
+    s += gz_align(realize_group_ws(F, R, L, npar, realize_merge_groups(F, R, (int)nch)));          // first merge stage
     s += 2 * gz_align((size_t)nch * F * 4);                  // dispatch plan, cost buckets
     s += gz_align((size_t)F * nt * 4);                       // tile costs
     return s + 512;
@@ -1387,7 +1388,7 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     A.p_ptot = (double*)p;        p += gz_align(pr * 8 * (size_t)npar);
     A.p_key = (uint64_t*)p;       p += gz_align(pr * 8 * (size_t)L);
     A.p_bin = (int32_t*)p;        p += gz_align(pr * 4 * (size_t)L);
-    void* group_ws = p;           p += gz_align(realize_group_ws(F, R, L, npar));
+    void* group_ws = p;           p += gz_align(realize_group_ws(F, R, L, npar, realize_merge_groups(F, R, A.nchunks)));
     A.plan = (int32_t*)p;         p += gz_align((size_t)A.nchunks * F * 4);
     A.plan_b = (int32_t*)p;       p += gz_align((size_t)A.nchunks * F * 4);
     A.tile_cost = (float*)p;
@@ -1427,7 +1428,8 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     }
     if (rc) return rc;
     return realize_merge_launch(h2fdf, par, order, B, F, R, L, mode, npar, A.nchunks, A.p_total, A.p_ptot, A.p_key,
-                                A.p_bin, hc2ss, ssidx, hc2bg, (npar > 0) ? bgpar : nullptr, group_ws, st);
+                                A.p_bin, hc2ss, ssidx, hc2bg, (npar > 0) ? bgpar : nullptr, group_ws,
+                                realize_merge_groups(F, R, A.nchunks), st);
 }
 
 extern "C" int hd_realize(const double* number, const double* h2fdf, const int64_t* order, int64_t B, int F, int R, int L,
