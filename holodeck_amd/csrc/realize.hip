@@ -18,6 +18,7 @@
 //     total - sum(selected h), which is exactly the reference's accounting
 //     (sum(n h) - max for ss_bg_hc; sum((n - taken) h) for the sorted walk,
 //     including its treatment of non-integer Normal draws).
+#include <algorithm>
 #include <type_traits>
 #include "common.hpp"
 #include "rng.hpp"
@@ -360,7 +361,7 @@ int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* 
 static int counts_chunk_bins(int64_t B, int F, int R) {
     const int64_t waves = cdiv((int64_t)F * R, 64);
     int64_t nch = cdiv(RZ_WAVES, waves);
-    nch = min(nch, min((int64_t)RZ_MAX_CHUNKS, cdiv(B, RZ_MIN_CHUNK)));
+    nch = std::min(nch, std::min((int64_t)RZ_MAX_CHUNKS, cdiv(B, RZ_MIN_CHUNK)));
     return (int)(cdiv(cdiv(B, nch), RZ_U) * RZ_U);
 }
 

@@ -49,7 +49,7 @@
 //                 sparse records (cumulative lambda); the tile's cost estimate;
 //   k_gz_plan  -- one workgroup: the draw workgroups' dispatch order, (chunk,
 //                 frequency) items by decreasing estimated cost;
-//   k_gz_draw  -- per (chunk of 8 tiles, frequency) workgroup, one realization
+//   k_gz_draw  -- per (chunk of up to 8 tiles, frequency) workgroup, one realization
 //                 per thread: tables of consecutive records are built in LDS
 //                 in batches that fit (a lane per short table, a 16-lane row
 //                 per mid-size table, a wave per long one); then every
@@ -62,13 +62,14 @@
 #include "common.hpp"
 #include "rng.hpp"
 #include "../../include/holohip.h"
+#include <algorithm>
 #include <mutex>
 
 namespace hd {
 
 constexpr int GZ_TILE = 512;          // bins per tile (prep workgroup size)
 constexpr int GZ_REC = GZ_TILE + 1;   // record slots per tile (+1 sparse pseudo-record)
-constexpr int GZ_TILES_PER_CHUNK = 8;    // items of 8 tiles: short enough to pack the GPU to its end
+constexpr int GZ_TPC_MAX = 8;         // tiles per (chunk, f) item, at most (gz_tpc chooses)
 constexpr int GZ_MAXBS = 512;         // draw workgroup: one realization per thread
 constexpr int GZ_BATCH_REC = 128;     // at most this many records per LDS batch (their headers are staged)
 constexpr int GZ_XCDS = 8;            // MI355X: 8 XCDs, workgroups dispatched round-robin
@@ -110,6 +111,8 @@ struct GapArgs {
     const double* par;      // (npar,B,F) or null
     int64_t B;
     int F, R, L, flags, npar, ntiles, nchunks, mode, cap;
+    int tpc;                // tiles per chunk
+    int big_nw;             // k_gz_big: waves of a group
     double thresh, tau;
     uint64_t seed;
     DRec* drec;             // (F, ntiles, GZ_REC)
@@ -390,12 +393,12 @@ __global__ void __launch_bounds__(GZ_PLAN_THREADS) k_gz_plan(GapArgs A) {
     __syncthreads();
     for (int it = tid; it < n; it += GZ_PLAN_THREADS) {
         const int f = it / A.nchunks, chunk = it - f * A.nchunks;
-        const int t0 = chunk * GZ_TILES_PER_CHUNK;
+        const int t0 = chunk * A.tpc;
         const float* tc = A.tile_cost + (int64_t)f * A.ntiles;
         double cost = 1.0;
 #pragma unroll
-        for (int k = 0; k < GZ_TILES_PER_CHUNK; k++)   // contiguous, every load issued first
-            cost += (t0 + k < A.ntiles) ? (double)tc[min(t0 + k, A.ntiles - 1)] : 0.0;
+        for (int k = 0; k < GZ_TPC_MAX; k++)   // contiguous, every load issued first
+            cost += (k < A.tpc && t0 + k < A.ntiles) ? (double)tc[min(t0 + k, A.ntiles - 1)] : 0.0;
         const int b = (int)fmin(fmax((double)(GZ_PLAN_BUCKETS - 1) - floor(4.0 * log2(cost)), 0.0),
                                 (double)(GZ_PLAN_BUCKETS - 1));
         A.plan_b[it] = b;
@@ -452,6 +455,9 @@ struct LoudList<HD_SEL_SORTED, LM> {
         for (int i = 0; i < LM; i++)
             if (i == L - 1) wk = k[i];
     }
+    __device__ __forceinline__ void merge(uint32_t key, int L) {   // an instance by its rank (none: 0xffffffff)
+        if (key < wk) insert((uint64_t)key, 0.0, L);
+    }
     __device__ __forceinline__ uint64_t key_at(int j) const {
         return k[j] == 0xffffffffu ? GZ_KEY_NONE : (uint64_t)k[j];
     }
@@ -492,9 +498,13 @@ struct LoudList {
         return (key < wk) || (key == wk && bin < wb);
     }
     __device__ __forceinline__ void insert(uint64_t word, double h, int L) {
+        insert_key(gz_hkey(h), (int32_t)(word >> 32), L);
+    }
+    __device__ __forceinline__ void merge(uint64_t key, int32_t bin, int L) {   // an instance as stored
+        if (key < wk || (key == wk && bin < wb)) insert_key(key, bin, L);
+    }
+    __device__ __forceinline__ void insert_key(uint64_t key, int32_t bin, int L) {
         if (gz_exact(LM)) L = LM;
-        uint64_t key = gz_hkey(h);
-        int32_t bin = (int32_t)(word >> 32);
 #pragma unroll
         for (int i = 0; i < LM; i++) {
             bool sw = (key < k[i]) || (key == k[i] && bin < b[i]);
@@ -673,6 +683,97 @@ __device__ __noinline__ void gz_build(gz_lds_u32* hi, double lam, int kb, int kt
         lo[e] = l;
     }
 }
+
+// One part of a long table, built by a wave: the counts [j_lo, j_hi) of the kb .. kt + n - 1 summed.
+// Where a batch holds fewer long tables than the workgroup has waves, each is cut into parts so
+// that every wave has one: a lane's serial recurrence, which the whole batch waits for, is then a
+// part's length / 64 instead of the table's.  The part's first pmf comes from the saddle-point form
+// (its own anchor: no product over the earlier parts).  gz_part_sum leaves the part's last running sum in
+// s_part as (first pmf of its last lane, that lane's relative sum, the carry into that lane);
+// gz_part_base of every later part sums these up, and leaves the part's largest value in s_part[3],
+// which the later parts' entries are raised to where rounding would put them below it (as gz_build
+// does between lanes), so the table is non-decreasing; gz_part_write then writes the entries.
+struct GzPart {
+    double pstart, carry, before;
+    int j0, m;       // this lane's counts
+};
+
+__device__ __noinline__ GzPart gz_part_sum(gz_lds_u32* hi, double lam, int kb, int kt, int n, double p0, int j_lo,
+                                           int j_hi, int lane, double* s_part) {
+    gz_lds_u32* lo = hi + n;
+    const int nb = j_hi - j_lo;
+    const int s = (nb + 63) >> 6;
+    GzPart P;
+    P.j0 = j_lo + lane * s;
+    P.m = min(max(j_hi - P.j0, 0), s);
+    const double kf = (double)(kb + P.j0);
+    const int jt = kt - kb - P.j0;
+    const double anchor = (j_lo == 0) ? p0 : gz_pmf_acc(lam, (double)(kb + j_lo));
+    double prod = 1.0, rel = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < P.m; j++) {
+        rel += prod;
+        if (j >= jt) {
+            hi[j - jt] = (uint32_t)__double2loint(rel);
+            lo[j - jt] = (uint32_t)__double2hiint(rel);
+        }
+        prod *= lam * gz_rcp(kf + (double)(j + 1));
+    }
+    P.pstart = anchor * gz_group_prev<64>(gz_group_scan<64>(prod, 1.0, GzMul()), 1.0);
+    P.carry = gz_group_prev<64>(gz_group_scan<64>(P.pstart * rel, 0.0, GzAdd()), 0.0);
+    if (P.m > 0 && P.j0 + P.m == j_hi) {   // the lane of the part's last count
+        s_part[0] = P.pstart;
+        s_part[1] = rel;
+        s_part[2] = P.carry;
+    }
+    return P;
+}
+
+// part: its index; s_part: the part sums of the table's part 0 (4 doubles each)
+__device__ __noinline__ void gz_part_base(gz_lds_u32* hi, int kb, int kt, int n, GzPart& P, int part, int lane,
+                                          double* s_part) {
+    const gz_lds_u32* lo = hi + n;
+    const int jt = kt - kb - P.j0;
+    double base = 0.0;
+    for (int q = 0; q < part; q++) base = __fma_rn(s_part[4 * q], s_part[4 * q + 1], base + s_part[4 * q + 2]);
+    P.carry += base;
+    // the lane's last value (the parked relative sum; none below the table)
+    const int e = P.m - 1 - jt;
+    const double ninf = -__builtin_inf();
+    double last = ninf;
+    if (P.m > 0 && e >= 0) last = __fma_rn(P.pstart, __hiloint2double((int)lo[e], (int)hi[e]), P.carry);
+    const double upto = gz_group_scan<64>(last, ninf, GzMax());
+    P.before = gz_group_prev<64>(upto, ninf);
+    if (lane == 63) s_part[4 * part + 3] = upto;
+}
+
+__device__ __noinline__ void gz_part_write(gz_lds_u32* hi, int kb, int kt, int n, GzPart P, int part,
+                                           const double* s_part) {
+    gz_lds_u32* lo = hi + n;
+    const int jt = kt - kb - P.j0;
+    double before = P.before;
+    for (int q = 0; q < part; q++) before = fmax(before, s_part[4 * q + 3]);
+#pragma unroll 4
+    for (int j = max(jt, 0); j < P.m; j++) {
+        const int e = j - jt;
+        const double r = __hiloint2double((int)lo[e], (int)hi[e]);
+        uint32_t h, l;
+        gz_fixed64(fmax(__fma_rn(P.pstart, r, P.carry), before), h, l);
+        hi[e] = h;
+        lo[e] = l;
+    }
+}
+
+// Parts of each of nl long tables for a workgroup of GZ_WAVES waves; below GZ_SPLIT_MIN counts
+// summed over them the parts' own anchors and scans cost more than the shorter recurrence gives.
+constexpr int GZ_WAVES = GZ_MAXBS / 64;
+#ifndef HD_GZ_SPLIT_MIN
+#define HD_GZ_SPLIT_MIN 2048
+#endif
+__device__ __forceinline__ int gz_parts(int nl, int lsum) {
+    return (nl > 0 && nl <= GZ_WAVES / 2 && lsum >= HD_GZ_SPLIT_MIN) ? GZ_WAVES / nl : 1;
+}
+__device__ __forceinline__ int gz_part_edge(int nb, int part, int parts) { return (int)((int64_t)nb * part / parts); }
 
 // Counts summed (kt + n - kb) up to which a table is built by a 16-lane row, four per wave;
 // longer tables take a whole wave.
@@ -972,6 +1073,8 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     __shared__ int s_nlarge;           // long tables of the batch (a wave each)
     __shared__ int s_nrow;             // mid-size tables (a 16-lane row each)
     __shared__ int s_nshort;           // short tables (a lane each)
+    __shared__ int s_lsum;             // counts summed over the long tables
+    __shared__ double s_part[GZ_WAVES][4];   // sums of the parts of split long tables
     __shared__ int s_large[GZ_BATCH_REC];
     __shared__ int s_row[GZ_BATCH_REC];
     __shared__ int s_short[GZ_BATCH_REC];
@@ -984,8 +1087,8 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int bs = blockDim.x;
     const int F = A.F, R = A.R, L = A.L;
-    const int t0 = chunk * GZ_TILES_PER_CHUNK;
-    const int t1 = min(t0 + GZ_TILES_PER_CHUNK, A.ntiles);
+    const int t0 = chunk * A.tpc;
+    const int t1 = min(t0 + A.tpc, A.ntiles);
     const int64_t pstride = (int64_t)F * A.ntiles * GZ_TILE;
     const uint32_t k0 = (uint32_t)A.seed, k1 = (uint32_t)(A.seed >> 32);
 
@@ -1025,6 +1128,7 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                     s_nlarge = 0;
                     s_nrow = 0;
                     s_nshort = 0;
+                    s_lsum = 0;
                 }
                 __syncthreads();   // the previous batch's draws are done with tab / scum
                 // one thread per record of the batch stages its header and lists its table as
@@ -1035,7 +1139,10 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                     const int nb = rec.kt + rec.n - rec.kb;
                     if (rec.n > 0 && nb <= GZ_SEQ_MAX) s_short[atomicAdd(&s_nshort, 1)] = tid;
                     else if (rec.n > 0 && nb <= HD_GZ_ROW_MAX) s_row[atomicAdd(&s_nrow, 1)] = tid;
-                    else if (rec.n > 0) s_large[atomicAdd(&s_nlarge, 1)] = tid;
+                    else if (rec.n > 0) {
+                        s_large[atomicAdd(&s_nlarge, 1)] = tid;
+                        atomicAdd(&s_lsum, nb);
+                    }
                 }
                 __syncthreads();
                 // build items handed out to the waves one at a time, the longest serial work
@@ -1043,7 +1150,29 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                 // 16-lane row each), then groups of 64 short tables (a lane each, one
                 // sequential pass), so that every lane a build occupies has work
                 {
-                    const int nl = s_nlarge, nr = s_nrow, nsh = s_nshort;
+                    int nl = s_nlarge;
+                    const int nr = s_nrow, nsh = s_nshort;
+                    const int parts = gz_parts(nl, s_lsum);
+                    if (parts > 1) {   // few long tables: cut so that each wave builds a part
+                        const int wv = tid >> 6;
+                        const BRec* rec = brec + s_large[min(wv / parts, nl - 1)];
+                        const int part = wv % parts, nb = rec->kt + rec->n - rec->kb;
+                        const bool on = wv < nl * parts;
+                        GzPart P;
+                        if (on)
+                            P = gz_part_sum((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kb, rec->kt, rec->n,
+                                            rec->p0, gz_part_edge(nb, part, parts), gz_part_edge(nb, part + 1, parts),
+                                            lane, s_part[wv]);
+                        __syncthreads();
+                        if (on)
+                            gz_part_base((gz_lds_u32*)(tab + 2 * rec->off), rec->kb, rec->kt, rec->n, P, part, lane,
+                                         s_part[wv - part]);
+                        __syncthreads();
+                        if (on)
+                            gz_part_write((gz_lds_u32*)(tab + 2 * rec->off), rec->kb, rec->kt, rec->n, P, part,
+                                          s_part[wv - part]);
+                        nl = 0;
+                    }
                     const int nrg = (nr + 3) >> 2, nsg = (nsh + 63) >> 6;
                     for (;;) {
                         int w = 0;
@@ -1129,68 +1258,202 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
 
 // Records without a table (lambda above the threshold or a window larger than
 // the LDS table): reload the chunk's partials, draw, store them back.
+//
+// Every (record, f, r) has its own stream, so a tile's records are shared by groups of waves: with R
+// realizations in nw = ceil(R / 64) waves, 8 / nw groups take the records in turn and the groups'
+// partials are added to the first one's at the end.  (A thread per realization walking every record
+// alone took 8.7 ms for 168,000 such records at R = 100, two waves per CU in flight.)  Per tile the
+// records are compacted in order and the factors of the rejection sampler that depend on lambda
+// alone are made once per record, a thread each, instead of by every realization.
+constexpr int GZ_BIG_THREADS = 512;
+struct GzBigRec {
+    double lam, h, loglam, a, b, vr, log_ia;
+    uint64_t word;
+    int i;   // position among the tile's dense records
+};
+
+// poisson_ptrs (rng.hpp) with its lambda-only factors given: the same operations on the same values
+__device__ __forceinline__ double gz_ptrs(Stream& st, const GzBigRec& q) {
+    const double lam = q.lam, b = q.b, a = q.a;
+    for (int it = 0; it < 100000; it++) {
+        double U = st.next() - 0.5;
+        double V = st.next();
+        double us = 0.5 - fabs(U);
+        double k = floor((2 * a / us + b) * U + lam + 0.43);
+        if ((us >= 0.07) && (V <= q.vr)) return k;
+        if ((k < 0) || ((us < 0.013) && (V > us))) continue;
+        if ((log(V) + q.log_ia - log(a / (us * us) + b)) <= (-lam + k * q.loglam - lgamma(k + 1.0))) return k;
+    }
+    return floor(lam);   // unreachable in practice; keeps the loop bounded
+}
+
 template <int MODE, int LM, int NP, bool REC>
-__global__ void __launch_bounds__(256) k_gz_big(GapArgs A) {
+__global__ void __launch_bounds__(GZ_BIG_THREADS) k_gz_big(GapArgs A) {
+    extern __shared__ double gz_big_lds[];   // a group's partials on their way to group 0
+    __shared__ GzBigRec s_rec[GZ_BIG_THREADS / 4];
+    __shared__ int s_cnt[GZ_BIG_THREADS / 64];
     const int f = blockIdx.y;
     const int chunk = blockIdx.x;
-    const int F = A.F, R = A.R, L = A.L;
-    const int t0 = chunk * GZ_TILES_PER_CHUNK;
-    const int t1 = min(t0 + GZ_TILES_PER_CHUNK, A.ntiles);
+    const int F = A.F, R = A.R, L = gz_exact(LM) ? LM : A.L;
+    const int t0 = chunk * A.tpc;
+    const int t1 = min(t0 + A.tpc, A.ntiles);
     const int64_t pstride = (int64_t)F * A.ntiles * GZ_TILE;
     int nbig = 0;
     for (int tile = t0; tile < t1; tile++) nbig += A.cnt[((int64_t)f * A.ntiles + tile) * 3 + 2];
     if (nbig == 0) return;
-    for (int r = threadIdx.x; r < R; r += blockDim.x) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // groups of nw waves (R above the workgroup's threads loops)
+    const int nw = A.big_nw;
+    const int ngroups = (GZ_BIG_THREADS / 64) / nw;
+    const int group = wv / nw;                       // waves past the last whole group only compact
+    const int rl = (wv - group * nw) * 64 + lane;    // realization within the group's span
+    const int span = nw * 64;
+    for (int rbase = 0; rbase < R; rbase += span) {
+        const int r = rbase + rl;
+        const bool on = group < ngroups && r < R;
         const int64_t pr = ((int64_t)f * A.nchunks + chunk) * R + r;
         Acc<MODE, LM, NP> acc;
-        acc.tot = A.p_total[pr];
+        acc.init();
+        if (on && group == 0) {
+            acc.tot = A.p_total[pr];
 #pragma unroll
-        for (int k = 0; k < NP; k++) acc.pt[k] = (k < A.npar) ? A.p_ptot[(int64_t)k * F * A.nchunks * R + pr] : 0.0;
-        if (MODE != HD_SEL_NONE) {
-            const int64_t o = ((pr / R) * L) * R + (pr % R);
-            acc.list.load(MODE == HD_SEL_SORTED ? (const uint64_t*)((const uint32_t*)A.p_key + o) : A.p_key + o,
-                          A.p_bin + o, L, R);
+            for (int k = 0; k < NP; k++) acc.pt[k] = (k < A.npar) ? A.p_ptot[(int64_t)k * F * A.nchunks * R + pr] : 0.0;
+            if (MODE != HD_SEL_NONE) {
+                const int64_t o = ((pr / R) * L) * R + (pr % R);
+                acc.list.load(MODE == HD_SEL_SORTED ? (const uint64_t*)((const uint32_t*)A.p_key + o) : A.p_key + o,
+                              A.p_bin + o, L, R);
+            }
         }
         for (int tile = t0; tile < t1; tile++) {
             const int64_t ft = (int64_t)f * A.ntiles + tile;
             if (A.cnt[ft * 3 + 2] == 0) continue;
             const int nd = A.cnt[ft * 3];
-            for (int i = 0; i < nd; i++) {
-                const DRec rec = A.drec[ft * GZ_REC + i];
-                if (rec.n != 0) continue;
-                const double n = gz_fallback((uint32_t)(rec.word >> 32), (uint32_t)f, (uint32_t)r, 3u, A.seed, rec.lam,
-                                             A.thresh);
-                acc.add(n, rec.h, rec.word, A.d_par + ft * GZ_TILE + i, pstride, A.npar, L);
-                if (REC) gz_record(A, rec.word, f, r, n, false);
+            // GZ_BIG_THREADS / 4 dense records at a time: those without a table, in order
+            for (int c = 0; c < nd; c += GZ_BIG_THREADS / 4) {
+                const int i = c + tid;
+                bool big = false;
+                GzBigRec q;
+                if (tid < GZ_BIG_THREADS / 4 && i < nd) {
+                    const DRec d = A.drec[ft * GZ_REC + i];
+                    big = d.n == 0;
+                    q.lam = d.lam;
+                    q.h = d.h;
+                    q.word = d.word;
+                    q.i = i;
+                }
+                const uint64_t mask = __ballot(big);
+                __syncthreads();   // the previous records' readers are done
+                if (lane == 0) s_cnt[wv] = __popcll(mask);
+                __syncthreads();
+                int off = 0, nb = 0;
+                for (int w = 0; w < GZ_BIG_THREADS / 256; w++) {
+                    if (w < wv) off += s_cnt[w];
+                    nb += s_cnt[w];
+                }
+                if (big) {
+                    const double slam = sqrt(q.lam);
+                    q.loglam = log(q.lam);
+                    q.b = 0.931 + 2.53 * slam;
+                    q.a = -0.059 + 0.02483 * q.b;
+                    q.log_ia = log(1.1239 + 1.1328 / (q.b - 3.4));
+                    q.vr = 0.9277 - 3.6224 / (q.b - 2);
+                    s_rec[off + __popcll(mask & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))))] = q;
+                }
+                __syncthreads();
+                if (on)
+                    for (int k = group; k < nb; k += ngroups) {
+                        const GzBigRec& s = s_rec[k];
+                        const uint32_t bin = (uint32_t)(s.word >> 32);
+                        double n;
+                        if (s.lam > A.thresh || s.lam < 10.0) {
+                            n = gz_fallback(bin, (uint32_t)f, (uint32_t)r, 3u, A.seed, s.lam, A.thresh);
+                        } else {
+                            Stream st;
+                            st.init(bin, (uint32_t)f, (uint32_t)r, 3u, A.seed);
+                            n = gz_ptrs(st, s);
+                        }
+                        acc.add(n, s.h, s.word, A.d_par + ft * GZ_TILE + s.i, pstride, A.npar, L);
+                        if (REC) gz_record(A, s.word, f, r, n, false);
+                    }
             }
         }
-        gz_store<MODE, LM, NP>(A, acc, pr);
+        // the groups' partials, one group at a time in order, into group 0's
+        for (int g = 1; g < ngroups; g++) {
+            double* s_tot = gz_big_lds;                       // span
+            double* s_pt = s_tot + span;                      // npar x span
+            uint64_t* s_key = (uint64_t*)(s_pt + (int64_t)A.npar * span);   // L x span: (bin << 32 | rank) word
+            __syncthreads();
+            if (group == g) {
+                s_tot[rl] = acc.tot;
+#pragma unroll
+                for (int k = 0; k < NP; k++)
+                    if (k < A.npar) s_pt[k * span + rl] = acc.pt[k];
+                if (MODE != HD_SEL_NONE) {
+#pragma unroll
+                    for (int j = 0; j < LM; j++)
+                        if (j < L) {
+                            if constexpr (MODE == HD_SEL_SORTED) ((uint32_t*)s_key)[j * span + rl] = acc.list.k32(j);
+                            else {
+                                s_key[j * span + rl] = acc.list.key_at(j);
+                                ((int32_t*)(s_key + (int64_t)L * span))[j * span + rl] = acc.list.bin_at(j, A.order);
+                            }
+                        }
+                }
+            }
+            __syncthreads();
+            if (on && group == 0) {
+                acc.tot += s_tot[rl];
+#pragma unroll
+                for (int k = 0; k < NP; k++)
+                    if (k < A.npar) acc.pt[k] += s_pt[k * span + rl];
+                if (MODE != HD_SEL_NONE)
+                    for (int j = 0; j < L; j++) {
+                        if constexpr (MODE == HD_SEL_SORTED)
+                            acc.list.merge(((const uint32_t*)s_key)[j * span + rl], L);
+                        else
+                            acc.list.merge(s_key[j * span + rl],
+                                           ((const int32_t*)(s_key + (int64_t)L * span))[j * span + rl], L);
+                    }
+            }
+        }
+        if (on && group == 0) gz_store<MODE, LM, NP>(A, acc, pr);
     }
 }
 
 // ---------------------------------------------------------------------------
 // hooks for tests: one CDF window built by one wave; draws from given words
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_cdf_table_hook(double lam, int cap, int* kn, uint64_t* cdf_out) {
+__global__ void __launch_bounds__(GZ_MAXBS) k_cdf_table_hook(double lam, int cap, int* kn, uint64_t* cdf_out) {
     extern __shared__ double hook_lds[];
+    __shared__ double s_part[GZ_WAVES][4];
     uint32_t* tab = (uint32_t*)hook_lds;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int kb, kt, n;
     gz_window(lam, cap, kb, kt, n);
-    if (n > 0) {   // the build the draw kernel uses for this length
-        if (kt + n - kb <= GZ_SEQ_MAX) {
-            if (lane == 0) gz_build_seq(tab, lam, kb, kt, n, gz_pmf_acc(lam, (double)kb));
-        } else if (kt + n - kb <= HD_GZ_ROW_MAX) {   // row 0 builds, rows 1-3 idle
+    if (n > 0) {   // the build the draw kernel uses for this length, alone in its batch
+        const int nb = kt + n - kb;
+        const double p0 = gz_pmf_acc(lam, (double)kb);
+        const int parts = gz_parts(1, nb);
+        if (nb <= GZ_SEQ_MAX) {
+            if (threadIdx.x == 0) gz_build_seq(tab, lam, kb, kt, n, p0);
+        } else if (nb <= HD_GZ_ROW_MAX) {   // row 0 builds, rows 1-3 idle
             const bool on = lane < 16;
-            gz_build<16>((gz_lds_u32*)tab, lam, on ? kb : 0, on ? kt : 0, on ? n : 0, gz_pmf_acc(lam, (double)kb),
-                         lane & 15);
-        } else {
-            gz_build<64>((gz_lds_u32*)tab, lam, kb, kt, n, gz_pmf_acc(lam, (double)kb), lane);
+            if (wv == 0)
+                gz_build<16>((gz_lds_u32*)tab, lam, on ? kb : 0, on ? kt : 0, on ? n : 0, p0, lane & 15);
+        } else if (parts > 1) {
+            GzPart P = gz_part_sum((gz_lds_u32*)tab, lam, kb, kt, n, p0, gz_part_edge(nb, wv, parts),
+                                   gz_part_edge(nb, wv + 1, parts), lane, s_part[wv]);
+            __syncthreads();
+            gz_part_base((gz_lds_u32*)tab, kb, kt, n, P, wv, lane, s_part[0]);
+            __syncthreads();
+            gz_part_write((gz_lds_u32*)tab, kb, kt, n, P, wv, s_part[0]);
+        } else if (wv == 0) {
+            gz_build<64>((gz_lds_u32*)tab, lam, kb, kt, n, p0, lane);
         }
     }
     __syncthreads();
-    for (int j = lane; j < n; j += 64) cdf_out[j] = ((uint64_t)tab[j] << 32) | tab[n + j];
-    if (lane == 0) {
+    for (int j = threadIdx.x; j < n; j += GZ_MAXBS) cdf_out[j] = ((uint64_t)tab[j] << 32) | tab[n + j];
+    if (threadIdx.x == 0) {
         kn[0] = kb;
         kn[1] = kt;
         kn[2] = n;
@@ -1277,9 +1540,17 @@ static_assert(3 * (GZ_DRAW_LDS + 2048) <= 160 * 1024, "three draw workgroups no 
 constexpr int GZ_HOOK_CAP_MAX = 8000;   // hd_poisson_cdf_table: 8-byte slots, 64000 B of LDS
 static_assert(GZ_HOOK_CAP_MAX * sizeof(double) <= 65536, "hook table above 64 KB");
 
-static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
+// Groups of the first merge stage: 8 with items of 8 tiles, by the chunk count with smaller ones.
+static int gz_groups(int F, int R, int nch, int tpc) {
+    if (tpc == GZ_TPC_MAX) return nch > 16 ? 8 : 0;
+    return realize_merge_groups(F, R, nch);
+}
+
+// Workspace of a call whose items have tpc tiles; key_bytes per partial list slot (4 for the
+// sorted walk's ranks, 12 for argmax's keys and bins).
+static size_t gz_need(int64_t B, int F, int R, int L, int npar, int tpc, int key_bytes) {
     const int64_t nt = cdiv(B, GZ_TILE);
-    const int64_t nch = cdiv(nt, GZ_TILES_PER_CHUNK);
+    const int64_t nch = cdiv(nt, tpc);
     const size_t slots = (size_t)F * nt * GZ_TILE;
     const size_t rslots = (size_t)F * nt * GZ_REC;
     const size_t pr = (size_t)F * nch * R;
@@ -1289,12 +1560,42 @@ static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
     s += gz_align((size_t)F * nt * 3 * 4);                 // counts
     s += 3 * gz_align(slots * 8);                          // sparse cum, h, word
     s += 2 * gz_align(slots * 8 * (size_t)npar);           // params
-    s += gz_align(pr * 8) + gz_align(pr * 8 * (size_t)npar) + gz_align(pr * 8 * (size_t)L) +
+    s += gz_align(pr * 8) + gz_align(pr * 8 * (size_t)npar) + gz_align(pr * (size_t)(key_bytes & ~7) * (size_t)L) +
          gz_align(pr * 4 * (size_t)L);
-    s += gz_align(realize_group_ws(F, R, L, npar, realize_merge_groups(F, R, (int)nch)));          // first merge stage
+    // first merge stage (room for 8 groups in any case)
+    s += gz_align(realize_group_ws(F, R, L, npar, std::max(8, gz_groups(F, R, (int)nch, tpc))));
     s += 2 * gz_align((size_t)nch * F * 4);                  // dispatch plan, cost buckets
     s += gz_align((size_t)F * nt * 4);                       // tile costs
     return s + 512;
+}
+
+// Tiles per item that the draw wants: 8 where that leaves at least GZ_MIN_ITEMS items (5 per
+// resident workgroup; larger items mean fewer partials to write and merge), else fewer: with 8
+// everywhere the 61 x 51 x 41 x 20 GW-driven grid had 600 items for 768 resident workgroups, the
+// longest 17.4 ms.
+constexpr int64_t GZ_MIN_ITEMS = 4096;
+static int gz_tpc_wanted(int64_t B, int F) {
+    int g = GZ_TPC_MAX;
+    while (g > 1 && cdiv(cdiv(B, GZ_TILE), g) * F < GZ_MIN_ITEMS) g >>= 1;
+    return g;
+}
+
+// The caller's workspace: what the wanted items take in any mode, except that a size served by the
+// fixed scratch of hd_realize_noalloc with items of 8 tiles stays within it.
+static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
+    const size_t most = gz_need(B, F, R, L, npar, GZ_TPC_MAX, 12);
+    const size_t want = gz_need(B, F, R, L, npar, gz_tpc_wanted(B, F), 12);
+    if (most > HD_NOALLOC_SCRATCH_BYTES) return std::max(most, want);
+    return std::max(most, std::min(want, (size_t)HD_NOALLOC_SCRATCH_BYTES));
+}
+
+// Tiles per item of a call: as wanted if the workspace of gz_ws holds its partials, else more.  (A
+// function of the sizes and mode alone, so that every entry point sums in the same order.)
+static int gz_tpc(int64_t B, int F, int R, int L, int npar, int mode) {
+    const size_t have = gz_ws(B, F, R, L, npar);
+    int g = gz_tpc_wanted(B, F);
+    while (g < GZ_TPC_MAX && gz_need(B, F, R, L, npar, g, mode == HD_SEL_SORTED ? 4 : 12) > have) g <<= 1;
+    return g;
 }
 
 template <int MODE, int LM, int NP, bool REC>
@@ -1305,7 +1606,18 @@ static int gz_launch_k(const GapArgs& A, dim3 grid, int bs, size_t lds, hipStrea
     }
     int rc = check_launch("k_gz_draw");
     if (rc) return rc;
-    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), grid, dim3(256), 0, st, A);
+    // groups of as few waves as hold the realizations, and LDS for one group's partials; one group of
+    // all waves where R fills them or the partials (many parameters and slots) would pass 48 KB
+    GapArgs Ab = A;
+    Ab.big_nw = (int)std::min((int64_t)GZ_BIG_THREADS / 64, cdiv(A.R, 64));
+    const size_t per = sizeof(double) * (1 + (size_t)A.npar) +
+                       (MODE == HD_SEL_SORTED ? sizeof(uint32_t) : sizeof(uint64_t) + sizeof(int32_t)) * (size_t)A.L;
+    size_t big_lds = per * Ab.big_nw * 64;
+    if (2 * Ab.big_nw > GZ_BIG_THREADS / 64 || big_lds > 48 * 1024) {
+        Ab.big_nw = GZ_BIG_THREADS / 64;
+        big_lds = 0;
+    }
+    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), grid, dim3(GZ_BIG_THREADS), big_lds, st, Ab);
     return check_launch("k_gz_big");
 }
 
@@ -1370,7 +1682,8 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     A.seed = seed;
     A.counts_out = counts_out;
     A.ntiles = (int)cdiv(B, GZ_TILE);
-    A.nchunks = (int)cdiv(A.ntiles, GZ_TILES_PER_CHUNK);
+    A.tpc = gz_tpc(B, F, R, L, npar, mode);
+    A.nchunks = (int)cdiv(A.ntiles, A.tpc);
     const size_t slots = (size_t)F * A.ntiles * GZ_TILE;
     const size_t rslots = (size_t)F * A.ntiles * GZ_REC;
     const size_t pr = (size_t)F * A.nchunks * R;
@@ -1386,9 +1699,9 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     A.sp_par = (double*)p;        p += gz_align(slots * 8 * (size_t)npar);
     A.p_total = (double*)p;       p += gz_align(pr * 8);
     A.p_ptot = (double*)p;        p += gz_align(pr * 8 * (size_t)npar);
-    A.p_key = (uint64_t*)p;       p += gz_align(pr * 8 * (size_t)L);
+    A.p_key = (uint64_t*)p;       p += gz_align(pr * (mode == HD_SEL_SORTED ? 0 : 8) * (size_t)L);   // sorted: ranks, in p_bin's room
     A.p_bin = (int32_t*)p;        p += gz_align(pr * 4 * (size_t)L);
-    void* group_ws = p;           p += gz_align(realize_group_ws(F, R, L, npar, realize_merge_groups(F, R, A.nchunks)));
+    void* group_ws = p;           p += gz_align(realize_group_ws(F, R, L, npar, std::max(8, gz_groups(F, R, A.nchunks, A.tpc))));
     A.plan = (int32_t*)p;         p += gz_align((size_t)A.nchunks * F * 4);
     A.plan_b = (int32_t*)p;       p += gz_align((size_t)A.nchunks * F * 4);
     A.tile_cost = (float*)p;
@@ -1429,7 +1742,7 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     if (rc) return rc;
     return realize_merge_launch(h2fdf, par, order, B, F, R, L, mode, npar, A.nchunks, A.p_total, A.p_ptot, A.p_key,
                                 A.p_bin, hc2ss, ssidx, hc2bg, (npar > 0) ? bgpar : nullptr, group_ws,
-                                realize_merge_groups(F, R, A.nchunks), st);
+                                gz_groups(F, R, A.nchunks, A.tpc), st);
 }
 
 extern "C" int hd_realize(const double* number, const double* h2fdf, const int64_t* order, int64_t B, int F, int R, int L,
@@ -1536,7 +1849,7 @@ extern "C" int hd_poisson_cdf_table(double lam, int cap, int* kb_kt_n, uint64_t*
         gz_window(lam, cap, kb, kt, n);
         if (n < 1) return set_error(HD_ERR_SIZE, "hd_poisson_cdf_table: table of lam=%g exceeds cap=%d", lam, cap);
     }
-    hipLaunchKernelGGL(k_cdf_table_hook, dim3(1), dim3(64), (size_t)cap * sizeof(double), (hipStream_t)stream, lam,
+    hipLaunchKernelGGL(k_cdf_table_hook, dim3(1), dim3(GZ_MAXBS), (size_t)cap * sizeof(double), (hipStream_t)stream, lam,
                        cap, kb_kt_n, cdf);
     return check_launch("k_cdf_table_hook");
 }
