@@ -20,6 +20,20 @@ _D = C.c_double
 _P = C.c_void_p
 _SZ = C.c_size_t
 
+MLP_MAX_LAYERS = 8
+_P8 = _P * MLP_MAX_LAYERS
+
+
+class MlpNet(C.Structure):
+    """hd_mlp_net."""
+    _fields_ = [("n_layers", _I32), ("sizes", _I32 * (MLP_MAX_LAYERS + 1)), ("w", _P8), ("b", _P8)]
+
+
+class MlpParams(C.Structure):
+    """hd_mlp_params."""
+    _fields_ = [(name, _P8) for name in ("w", "b", "wb", "mw", "vw", "mb", "vb", "dw", "db")]
+
+
 # name -> (restype, argtypes)
 SIGNATURES = {
     "hd_last_error": (C.c_char_p, []),
@@ -69,6 +83,11 @@ SIGNATURES = {
     "hd_mlp_colsum_bf16": (_I32, [_P, _I32, _I32, _P, _P]),
     "hd_mlp_mse": (_I32, [_P, _P, _I64, _P, _P, _P]),
     "hd_mlp_adam": (_I32, [_I64, _P, _P, _P, _P, C.c_float, C.c_float, C.c_float, C.c_float, _I32, _P, _P]),
+    "hd_mlp_fused": (_I32, [_P]),
+    "hd_mlp_forward": (_I32, [_P, _P, _P, _P, _I32, _P, _P, _P]),
+    "hd_mlp_train_workspace_size": (_SZ, [_P, _I32]),
+    "hd_mlp_train_step": (_I32, [_P, _P, _P, _P, _P, _I32, _P, _P, _I32, C.c_float, C.c_float, C.c_float, C.c_float,
+                                 _I32, _P, _SZ, _P]),
     "hd_gwb_ideal_workspace_size": (_SZ, []),
     "hd_gwb_ideal": (_I32, [_P, _P, _P, _I32, _P, _I32, _P, _I32, _I32, _P, _I32, _D, _D, _D, _I32, _P, _P, _SZ, _P]),
     "hd_eccen_workspace_size": (_SZ, [_I32, _I32, _I32]),

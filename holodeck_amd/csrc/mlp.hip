@@ -14,25 +14,15 @@
 //
 // MFMA 16x16x32 operand layout (lane l of 64): A row l%16, k 8*(l/16)..+7;
 // B column l%16, k 8*(l/16)..+7; accumulator column l%16, rows 4*(l/16)..+3.
-#include "common.hpp"
+#include "mlp.hpp"
 #include "../../include/holohip.h"
 
 namespace hd {
-
-typedef __bf16 bf16;
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 constexpr int MT = 64;       // tile M
 constexpr int NT = 64;       // tile N
 constexpr int KT = 32;       // tile K
 constexpr int KP = KT + 8;   // padded LDS row (bf16): 80 bytes, keeps 16-byte alignment
-
-__device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
-__device__ __forceinline__ float silu_grad(float z) {
-    const float s = 1.0f / (1.0f + __expf(-z));
-    return s * (1.0f + z * (1.0f - s));
-}
 
 // Epilogues
 //   HD_MLP_EPI_STORE      out_f32[m, n] = acc (+ bias[n])

@@ -15,6 +15,8 @@ buffers only.
 Outside the training box, or when asked to judge, the plain GPU SAM computes
 the spectrum (:class:`SurrogateWithFallback`).
 """
+import ctypes as C
+
 import numpy as np
 import torch
 
@@ -77,6 +79,17 @@ class MLPSurrogate:
         return np.all((x >= 0.0) & (x <= 1.0), axis=-1)
 
     # ---- device passes ----
+    def _net(self):
+        """This network for the whole-pass kernels, or None where they do not take its shape (then the
+        layers run one by one)."""
+        if self.nlayers > _lib.MLP_MAX_LAYERS:
+            return None
+        net = _lib.MlpNet(n_layers=self.nlayers)
+        net.sizes[:self.nlayers + 1] = self.sizes
+        for l in range(self.nlayers):
+            net.w[l], net.b[l] = D.ptr(self.Wb[l]), D.ptr(self.b[l])
+        return net if _lib.size("hd_mlp_fused", C.addressof(net)) else None
+
     def _forward(self, xb, keep):
         """xb: (M, n_in) bf16 device.  Returns output f32 (M, n_out) and, if keep, per-layer (z f32, h bf16)."""
         st = D.stream_ptr()
@@ -135,8 +148,16 @@ class MLPSurrogate:
 
     def loss_and_grads(self, X01, Yn):
         """Device loss (MSE on standardised targets) and gradients for one batch; X01, Yn numpy or tensors."""
-        xb = D.to_dev(np.asarray(X01, dtype=np.float32), dtype=torch.float32).to(torch.bfloat16).contiguous()
+        x = D.to_dev(np.asarray(X01, dtype=np.float32), dtype=torch.float32)
         t = D.to_dev(np.asarray(Yn, dtype=np.float32), dtype=torch.float32)
+        step = _TrainStep.of(self, x, t, x.shape[0])
+        if step is not None:
+            loss = torch.zeros(1, dtype=torch.float32, device=x.device)
+            y = _f32((x.shape[0], self.sizes[-1]))
+            grads = [(torch.empty_like(W), torch.empty_like(b)) for W, b in zip(self.W, self.b)]
+            step(None, x.shape[0], loss, y=y, grads=grads)
+            return loss, grads, y
+        xb = x.to(torch.bfloat16).contiguous()
         y, cache = self._forward(xb, keep=True)
         dy = _bf16(y.shape)
         loss = torch.zeros(1, dtype=torch.float32, device=y.device)
@@ -164,6 +185,7 @@ class MLPSurrogate:
         S = X.shape[0]
         gen = torch.Generator(device="cpu").manual_seed(seed)
         hist = []
+        step = _TrainStep.of(self, X01, Yn, min(batch, S))
         for ep in range(epochs):
             lr_ep = lr if lr_min is None else lr_min + 0.5 * (lr - lr_min) * (1.0 + np.cos(np.pi * ep / epochs))
             perm = torch.randperm(S, generator=gen).to(X01.device)
@@ -171,6 +193,10 @@ class MLPSurrogate:
             nb = 0
             for s0 in range(0, S - batch + 1 if S >= batch else 1, batch):
                 idx = perm[s0:s0 + batch]
+                if step is not None:
+                    step(idx, idx.numel(), tot, lr=lr_ep)
+                    nb += 1
+                    continue
                 xb = X01[idx].to(torch.bfloat16).contiguous()
                 t = Yn[idx].contiguous()
                 y, cache = self._forward(xb, keep=True)
@@ -185,6 +211,13 @@ class MLPSurrogate:
 
     def predict_device(self, X01_bf16):
         """Standardised outputs (M, n_out) f32 for device inputs already in [0, 1] (bf16)."""
+        net = self._net()
+        if net is not None and X01_bf16.dtype == torch.bfloat16 and X01_bf16.dim() == 2 and X01_bf16.shape[0] > 0 \
+                and X01_bf16.shape[1] == self.sizes[0]:
+            y = _f32((X01_bf16.shape[0], self.sizes[-1]))
+            _lib.call("hd_mlp_forward", C.addressof(net), D.ptr(X01_bf16), None, None, y.shape[0], D.ptr(y), None,
+                      D.stream_ptr())
+            return y
         y, _ = self._forward(X01_bf16, keep=False)
         return y
 
@@ -218,12 +251,67 @@ class MLPSurrogate:
 
     def predict(self, X, chunk=1 << 17):
         """log10 h_c percentile spectra (M, n_out) for parameters X (M, n_in)."""
+        X = np.asarray(X, dtype=float)
+        net = self._net()
+        if net is not None and X.ndim == 2 and X.shape[0] > 0 and X.shape[1] == self.sizes[0]:
+            # scaling to and from the training box on the device: the same double operations
+            scale = D.to_dev(np.concatenate([np.broadcast_to(v, n) for v, n in (
+                (self.x_lo, self.sizes[0]), (np.subtract(self.x_hi, self.x_lo), self.sizes[0]),
+                (self.y_std, self.sizes[-1]), (self.y_mean, self.sizes[-1]))]).astype(float, copy=False))
+            out = np.empty((X.shape[0], self.sizes[-1]))
+            for s0 in range(0, X.shape[0], chunk):
+                raw = D.to_dev(X[s0:s0 + chunk])
+                y = D.empty((raw.shape[0], self.sizes[-1]))
+                _lib.call("hd_mlp_forward", C.addressof(net), None, D.ptr(raw), D.ptr(scale), y.shape[0], None,
+                          D.ptr(y), D.stream_ptr())
+                out[s0:s0 + chunk] = D.to_host(y)
+            return out
         X01 = np.asarray(self._x01(X), dtype=np.float32)
         out = []
         for s0 in range(0, X01.shape[0], chunk):
             xb = D.to_dev(X01[s0:s0 + chunk], dtype=torch.float32).to(torch.bfloat16).contiguous()
             out.append(D.to_host(self.predict_device(xb)).astype(float))
         return np.concatenate(out) * self.y_std + self.y_mean
+
+
+class _TrainStep:
+    """Batches of a network's training on the whole-pass kernels (hd_mlp_train_step), with the
+    workspace of one batch."""
+
+    @classmethod
+    def of(cls, model, X, T, rows):
+        """For device inputs X (S, n_in) and targets T (S, n_out) f32, batches of at most ``rows``; None
+        where the kernels do not take the network or the arrays do not fit it."""
+        net = model._net()
+        if (net is None or model.sizes[-1] > 256 or rows < 1 or X.shape[1:] != (model.sizes[0],)
+                or T.shape != (X.shape[0], model.sizes[-1])):
+            return None
+        return cls(model, net, X, T, rows)
+
+    def __init__(self, model, net, X, T, rows):
+        self.model, self.net, self.X, self.T, self.rows = model, net, X, T, rows
+        self.ws = D.workspace(_lib.size("hd_mlp_train_workspace_size", C.addressof(net), rows))
+        self.par = _lib.MlpParams()
+        for l in range(model.nlayers):
+            for name, ts in (("w", model.W), ("b", model.b), ("wb", model.Wb), ("mw", model.mW), ("vw", model.vW),
+                             ("mb", model.mb), ("vb", model.vb)):
+                getattr(self.par, name)[l] = D.ptr(ts[l])
+        self.fresh = True
+
+    def __call__(self, idx, rows, loss, lr=0.0, y=None, grads=None, b1=0.9, b2=0.999, eps=1e-8):
+        """One batch: rows ``idx`` (device int64; None: the first ``rows``) with an Adam step, or, with
+        ``grads``, the gradients alone; adds the mean squared error to ``loss``."""
+        par = self.par
+        if grads is None:
+            self.model.step += 1
+        else:
+            par = _lib.MlpParams()
+            for l, (dW, db) in enumerate(grads):
+                par.dw[l], par.db[l] = D.ptr(dW), D.ptr(db)
+        _lib.call("hd_mlp_train_step", C.addressof(self.net), C.addressof(par), D.ptr(self.X), D.ptr(self.T),
+                  D.ptr(idx), rows, D.ptr(loss), D.ptr(y), int(self.fresh), lr, b1, b2, eps, max(self.model.step, 1),
+                  D.ptr(self.ws), self.ws.numel(), D.stream_ptr())
+        self.fresh = False
 
 
 class SurrogateWithFallback:

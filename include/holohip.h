@@ -322,6 +322,39 @@ int hd_mlp_adam(int64_t n, float *w, const float *g, float *m, float *v, float l
                 int step, void *w_bf16, void *stream);
 int hd_f32_to_bf16(const float *a, int64_t n, void *b, void *stream);
 
+/* Whole passes of a network whose hidden layers have a multiple of 32 units, at most 256, and whose
+ * input has at most 256 (hd_mlp_fused tells: 1 yes, 0 no; others take the calls above).  The layers
+ * are the same products in the same order as hd_mlp_gemm_bf16 makes them, with the activations of a
+ * block of rows kept on chip. */
+#define HD_MLP_MAX_LAYERS 8
+typedef struct {
+    int n_layers;                             /* 1 .. HD_MLP_MAX_LAYERS */
+    int sizes[HD_MLP_MAX_LAYERS + 1];         /* input, hidden..., output */
+    const void *w[HD_MLP_MAX_LAYERS];         /* bf16 (out, in) */
+    const float *b[HD_MLP_MAX_LAYERS];        /* (out) */
+} hd_mlp_net;
+int hd_mlp_fused(const hd_mlp_net *net);
+/* Inference over M rows.  Input: x (M, in) bf16, or x = NULL and raw (M, in) doubles with scale
+ * holding [low (in), width (in)], the row then being bf16((raw - low) / width) rounded through FP32.
+ * Output: y (M, out) FP32, or y = NULL and out (M, out) doubles y * spread + centre with scale going
+ * on [.., spread (out), centre (out)].  scale: 2 in + 2 out doubles, read for raw and out only. */
+int hd_mlp_forward(const hd_mlp_net *net, const void *x, const double *raw, const double *scale, int M, float *y,
+                   double *out, void *stream);
+/* One training batch: forward, mean squared error (added to *loss), gradients, and, with w[0] set, an
+ * Adam step (step >= 1) on the FP32 masters with their bf16 copies.  Row m of the batch is row
+ * idx[m] of X (rows, in) and T (rows, out), FP32 (idx NULL: row m).  y (M, out), dw/db: written when
+ * not NULL.  rebuild != 0: the weights changed since this workspace's last step (or it is new). */
+typedef struct {
+    float *w[HD_MLP_MAX_LAYERS], *b[HD_MLP_MAX_LAYERS];
+    void *wb[HD_MLP_MAX_LAYERS];
+    float *mw[HD_MLP_MAX_LAYERS], *vw[HD_MLP_MAX_LAYERS], *mb[HD_MLP_MAX_LAYERS], *vb[HD_MLP_MAX_LAYERS];
+    float *dw[HD_MLP_MAX_LAYERS], *db[HD_MLP_MAX_LAYERS];
+} hd_mlp_params;
+size_t hd_mlp_train_workspace_size(const hd_mlp_net *net, int M);
+int hd_mlp_train_step(const hd_mlp_net *net, const hd_mlp_params *par, const float *X, const float *T,
+                      const int64_t *idx, int M, float *loss, float *y, int rebuild, float lr, float b1, float b2,
+                      float eps, int step, void *workspace, size_t ws_bytes, void *stream);
+
 /* ------------------------------------------------------------------------
  * Eccentric SAM GWB over one eccentricity evolution e(a) shared by all binaries.
  * Inputs as the reference's Cython signatures: ndens (M,Q,Z) at the grid nodes
