@@ -174,14 +174,16 @@ class MLPSurrogate:
         (continued training).
         """
         X = np.asarray(X, dtype=float)
-        Y = np.asarray(Y, dtype=float)
+        Yn = D.to_dev(np.asarray(Y, dtype=float))
         if rescale:
             self.x_lo = X.min(axis=0) if x_lo is None else np.asarray(x_lo, float)
             self.x_hi = X.max(axis=0) if x_hi is None else np.asarray(x_hi, float)
-            self.y_mean = Y.mean(axis=0)
-            self.y_std = np.maximum(Y.std(axis=0), 1e-6)
+            mean, std = Yn.mean(dim=0), Yn.std(dim=0, unbiased=False).clamp(min=1e-6)
+            self.y_mean, self.y_std = D.to_host(mean), D.to_host(std)
+        else:
+            mean, std = D.to_dev(self.y_mean), D.to_dev(self.y_std)
         X01 = torch.as_tensor(self._x01(X), dtype=torch.float32).to(D.require_device())
-        Yn = torch.as_tensor((Y - self.y_mean) / self.y_std, dtype=torch.float32).to(D.require_device())
+        Yn = ((Yn - mean) / std).to(torch.float32)
         S = X.shape[0]
         gen = torch.Generator(device="cpu").manual_seed(seed)
         hist = []
@@ -255,16 +257,23 @@ class MLPSurrogate:
         net = self._net()
         if net is not None and X.ndim == 2 and X.shape[0] > 0 and X.shape[1] == self.sizes[0]:
             # scaling to and from the training box on the device: the same double operations
-            scale = D.to_dev(np.concatenate([np.broadcast_to(v, n) for v, n in (
-                (self.x_lo, self.sizes[0]), (np.subtract(self.x_hi, self.x_lo), self.sizes[0]),
-                (self.y_std, self.sizes[-1]), (self.y_mean, self.sizes[-1]))]).astype(float, copy=False))
-            out = np.empty((X.shape[0], self.sizes[-1]))
+            n_in, n_out = self.sizes[0], self.sizes[-1]
+            scale = np.empty(2 * (n_in + n_out))
+            scale[:n_in], scale[n_in:2 * n_in] = self.x_lo, np.subtract(self.x_hi, self.x_lo)
+            scale[2 * n_in:-n_out], scale[-n_out:] = self.y_std, self.y_mean
+            out = np.empty((X.shape[0], n_out))
+            one = X.nbytes <= D.STAGE_MAX_BYTES // 2 and X.shape[0] <= chunk
+            if one:      # a small call: the scaling and the rows in one upload
+                up = D.to_dev(np.concatenate([scale, X.ravel()]))
+                scale, X = up[:scale.size], up[scale.size:].view(X.shape)
+            else:
+                scale = D.to_dev(scale)
             for s0 in range(0, X.shape[0], chunk):
-                raw = D.to_dev(X[s0:s0 + chunk])
-                y = D.empty((raw.shape[0], self.sizes[-1]))
+                raw = X if one else D.to_dev(X[s0:s0 + chunk])
+                y = D.empty((raw.shape[0], n_out))
                 _lib.call("hd_mlp_forward", C.addressof(net), None, D.ptr(raw), D.ptr(scale), y.shape[0], None,
                           D.ptr(y), D.stream_ptr())
-                out[s0:s0 + chunk] = D.to_host(y)
+                D.to_host(y, out=out[s0:s0 + chunk])
             return out
         X01 = np.asarray(self._x01(X), dtype=np.float32)
         out = []
