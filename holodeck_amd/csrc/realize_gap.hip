@@ -112,7 +112,6 @@ struct GapArgs {
     int64_t B;
     int F, R, L, flags, npar, ntiles, nchunks, mode, cap;
     int tpc;                // tiles per chunk
-    int big_nw;             // k_gz_big: waves of a group
     double thresh, tau;
     uint64_t seed;
     DRec* drec;             // (F, ntiles, GZ_REC)
@@ -455,9 +454,6 @@ struct LoudList<HD_SEL_SORTED, LM> {
         for (int i = 0; i < LM; i++)
             if (i == L - 1) wk = k[i];
     }
-    __device__ __forceinline__ void merge(uint32_t key, int L) {   // an instance by its rank (none: 0xffffffff)
-        if (key < wk) insert((uint64_t)key, 0.0, L);
-    }
     __device__ __forceinline__ uint64_t key_at(int j) const {
         return k[j] == 0xffffffffu ? GZ_KEY_NONE : (uint64_t)k[j];
     }
@@ -498,13 +494,9 @@ struct LoudList {
         return (key < wk) || (key == wk && bin < wb);
     }
     __device__ __forceinline__ void insert(uint64_t word, double h, int L) {
-        insert_key(gz_hkey(h), (int32_t)(word >> 32), L);
-    }
-    __device__ __forceinline__ void merge(uint64_t key, int32_t bin, int L) {   // an instance as stored
-        if (key < wk || (key == wk && bin < wb)) insert_key(key, bin, L);
-    }
-    __device__ __forceinline__ void insert_key(uint64_t key, int32_t bin, int L) {
         if (gz_exact(LM)) L = LM;
+        uint64_t key = gz_hkey(h);
+        int32_t bin = (int32_t)(word >> 32);
 #pragma unroll
         for (int i = 0; i < LM; i++) {
             bool sw = (key < k[i]) || (key == k[i] && bin < b[i]);
@@ -1030,17 +1022,6 @@ __device__ __forceinline__ GzTab gz_tab_rec(const uint32_t* tab, const DRec& d, 
     return t;
 }
 
-// Counts without a table: Normal above the threshold, inversion below 10,
-// PTRS otherwise; stream (a, f, r, tag).
-__device__ __forceinline__ double gz_fallback(uint32_t a, uint32_t f, uint32_t r, uint32_t tag, uint64_t seed,
-                                              double lam, double thresh) {
-    Stream st;
-    st.init(a, f, r, tag, seed);
-    if (lam > thresh) return normal_count(st, lam);
-    if (lam < 10.0) return poisson_inversion(st.next(), lam, -expm1(-lam), exp(-lam));
-    return poisson_ptrs(st, lam);
-}
-
 template <int MODE, int LM, int NP>
 __device__ __forceinline__ void gz_store(const GapArgs& A, const Acc<MODE, LM, NP>& acc, int64_t pr) {
     const int F = A.F, R = A.R, L = gz_exact(LM) ? LM : A.L;
@@ -1259,42 +1240,146 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
 // Records without a table (lambda above the threshold or a window larger than
 // the LDS table): reload the chunk's partials, draw, store them back.
 //
-// Every (record, f, r) has its own stream, so a tile's records are shared by groups of waves: with R
-// realizations in nw = ceil(R / 64) waves, 8 / nw groups take the records in turn and the groups'
-// partials are added to the first one's at the end.  (A thread per realization walking every record
-// alone took 8.7 ms for 168,000 such records at R = 100, two waves per CU in flight.)  Per tile the
-// records are compacted in order and the factors of the rejection sampler that depend on lambda
-// alone are made once per record, a thread each, instead of by every realization.
-constexpr int GZ_BIG_THREADS = 512;
+// Every (record, f, r) has its own stream, so the draws of a round -- as many records of a tile as give
+// GZ_BIG_PAIRS of them -- are spread evenly over the lanes whatever R is, and their counts put in LDS;
+// then a thread per realization adds them up in record order.  The rejection sampler accepts four
+// draws of five by a cheap test; the others need two logarithms and a log-gamma, which a wave that
+// keeps a lane per draw executes for all its lanes almost every time.  A wave therefore sets such
+// draws aside in a queue and evaluates 64 of them at once, and likewise collects the rejected ones for
+// their next attempt (attempt i of a stream is Philox block i, so a draw's state is its number and i).
+// The factors that depend on lambda alone are made once per record.  Bound by VALU issue.  (Eccentric
+// realizations, 52,111 nodes x 600 columns x 100, 8.3 million such records: 66.7 ms with a thread per
+// realization, 36.1 with the records shared by groups of waves and a lane per draw, 12.8 so; at
+// most 168 registers, so that the three workgroups the LDS holds fit: 26.7 with the compiler free.)
+constexpr int GZ_BIG_THREADS = 256;
+constexpr int GZ_BIG_WAVES = GZ_BIG_THREADS / 64;
+constexpr int GZ_BIG_RECS = 128;     // records of a round, at most
+constexpr int GZ_BIG_PAIRS = 3072;   // (record, realization) draws of a round, at most
+constexpr int GZ_BIG_SLOW = 128;     // a wave's draws waiting for the exact test: below 64, plus 64 more
+constexpr int GZ_BIG_AGAIN = 192;    // and for another attempt: below 64, plus 64 from either test
 struct GzBigRec {
     double lam, h, loglam, a, b, vr, log_ia;
     uint64_t word;
     int i;   // position among the tile's dense records
 };
 
-// poisson_ptrs (rng.hpp) with its lambda-only factors given: the same operations on the same values
-__device__ __forceinline__ double gz_ptrs(Stream& st, const GzBigRec& q) {
-    const double lam = q.lam, b = q.b, a = q.a;
-    for (int it = 0; it < 100000; it++) {
-        double U = st.next() - 0.5;
-        double V = st.next();
-        double us = 0.5 - fabs(U);
-        double k = floor((2 * a / us + b) * U + lam + 0.43);
-        if ((us >= 0.07) && (V <= q.vr)) return k;
-        if ((k < 0) || ((us < 0.013) && (V > us))) continue;
-        if ((log(V) + q.log_ia - log(a / (us * us) + b)) <= (-lam + k * q.loglam - lgamma(k + 1.0))) return k;
+// A wave's queues; an entry: pair | attempt << 12
+struct GzBigQueue {
+    double k[GZ_BIG_SLOW], v[GZ_BIG_SLOW], us[GZ_BIG_SLOW];
+    uint32_t slow[GZ_BIG_SLOW], again[GZ_BIG_AGAIN];
+};
+static_assert(GZ_BIG_PAIRS <= 4096, "pair number in 12 bits");
+constexpr int GZ_BIG_TRIES = 100000;   // attempts of a draw: unreachable in practice, keeps the loop bounded
+
+// LDS written by a wave's lanes is read by others of the same wave after this (its LDS operations
+// complete in order; the compiler must not move them across)
+__device__ __forceinline__ void gz_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ int gz_below(uint64_t mask, int lane) {   // set bits below this lane's
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// The counts of one round's pairs [0, npairs), pair = record * rb + (r - rbase), into s_n; the wave takes
+// pairs wave * 64 + lane, + GZ_BIG_THREADS, ...  The tests are those of the
+// transformed rejection PTRS (W. Hoermann, Insurance: Mathematics and Economics 12, 1993), lambda >= 10.
+__device__ __forceinline__ void gz_big_draw(const GapArgs& A, const GzBigRec* s_rec, GzBigQueue& Q, double* s_n,
+                                            int npairs, int rb, int rbase, int f, int wv, int lane) {
+    const float inv_rb = 1.0f / (float)rb;
+    const uint32_t k0 = (uint32_t)A.seed, k1 = (uint32_t)(A.seed >> 32);
+    int next = wv * 64, nslow = 0, nagain = 0;
+    for (;;) {
+        const bool fresh = next < npairs;
+        if (nslow >= 64 || (!fresh && nagain == 0 && nslow > 0)) {   // exact tests, the last entries
+            const int n = min(nslow, 64), e = nslow - n + lane;
+            nslow -= n;
+            bool again = false;
+            uint32_t id = 0;
+            gz_wave_sync();
+            if (lane < n) {
+                id = Q.slow[e];
+                const double k = Q.k[e], V = Q.v[e], us = Q.us[e];
+                const GzBigRec& q = s_rec[(int)(((float)(id & 4095u) + 0.5f) * inv_rb)];
+                const double lam = q.lam, a = q.a, b = q.b;
+                again = !((log(V) + q.log_ia - log(a / (us * us) + b)) <= (-lam + k * q.loglam - lgamma(k + 1.0)));
+                if (!again) s_n[id & 4095u] = k;
+            }
+            const uint64_t m = __ballot(again);
+            gz_wave_sync();
+            if (again) Q.again[nagain + gz_below(m, lane)] = id + 4096u;
+            nagain += __popcll(m);
+            continue;
+        }
+        // an attempt: of draws set back if there are 64 (or nothing new), else of new ones
+        bool on;
+        uint32_t id;
+        if (nagain >= 64 || (!fresh && nagain > 0)) {
+            const int n = min(nagain, 64);
+            nagain -= n;
+            on = lane < n;
+            gz_wave_sync();
+            id = on ? Q.again[nagain + lane] : 0u;
+        } else if (fresh) {
+            on = next + lane < npairs;
+            id = (uint32_t)(next + lane);
+            next += GZ_BIG_THREADS;
+        } else {
+            break;
+        }
+        bool slow = false, again = false;
+        double k = 0.0, V = 0.0, us = 0.0;
+        if (on) {
+            const int pair = (int)(id & 4095u), it = (int)(id >> 12);
+            const int j = (int)(((float)pair + 0.5f) * inv_rb);   // exact: pair below 2^12
+            const uint32_t r = (uint32_t)(rbase + pair - j * rb);
+            const GzBigRec& q = s_rec[j];
+            const double lam = q.lam;
+            const uint32_t bin = (uint32_t)(q.word >> 32);
+            if (lam > A.thresh || lam < 10.0) {
+                Stream st;
+                st.init(bin, (uint32_t)f, r, 3u, A.seed);
+                s_n[pair] = (lam > A.thresh) ? normal_count(st, lam)
+                                             : poisson_inversion(st.next(), lam, -expm1(-lam), exp(-lam));
+            } else if (it >= GZ_BIG_TRIES) {
+                s_n[pair] = floor(lam);
+            } else {
+                const U4 w = philox4x32_10(U4{bin, (uint32_t)f, r, (3u << 16) + (uint32_t)it}, k0, k1);
+                const double U = u53(w.x, w.y) - 0.5;
+                V = u53(w.z, w.w);
+                us = 0.5 - fabs(U);
+                k = floor((2 * q.a / us + q.b) * U + lam + 0.43);
+                if ((us >= 0.07) && (V <= q.vr)) s_n[pair] = k;
+                else if ((k < 0) || ((us < 0.013) && (V > us))) again = true;
+                else slow = true;
+            }
+        }
+        const uint64_t ms = __ballot(slow), ma = __ballot(again);
+        gz_wave_sync();
+        if (slow) {
+            const int e = nslow + gz_below(ms, lane);
+            Q.slow[e] = id;
+            Q.k[e] = k;
+            Q.v[e] = V;
+            Q.us[e] = us;
+        }
+        if (again) Q.again[nagain + gz_below(ma, lane)] = id + 4096u;
+        nslow += __popcll(ms);
+        nagain += __popcll(ma);
     }
-    return floor(lam);   // unreachable in practice; keeps the loop bounded
 }
 
 template <int MODE, int LM, int NP, bool REC>
-__global__ void __launch_bounds__(GZ_BIG_THREADS) k_gz_big(GapArgs A) {
-    extern __shared__ double gz_big_lds[];   // a group's partials on their way to group 0
-    __shared__ GzBigRec s_rec[GZ_BIG_THREADS / 4];
-    __shared__ int s_cnt[GZ_BIG_THREADS / 64];
+__global__ void __launch_bounds__(GZ_BIG_THREADS, 3) k_gz_big(GapArgs A) {
+    __shared__ GzBigRec s_rec[GZ_BIG_RECS];
+    __shared__ double s_n[GZ_BIG_PAIRS];
+    __shared__ GzBigQueue s_q[GZ_BIG_WAVES];
+    __shared__ int s_cnt[GZ_BIG_WAVES];
+    __shared__ uint16_t s_list[GZ_TILE];   // the tile's records without a table, in order
     const int f = blockIdx.y;
     const int chunk = blockIdx.x;
-    const int F = A.F, R = A.R, L = gz_exact(LM) ? LM : A.L;
+    const int F = A.F, R = A.R, L = A.L;
     const int t0 = chunk * A.tpc;
     const int t1 = min(t0 + A.tpc, A.ntiles);
     const int64_t pstride = (int64_t)F * A.ntiles * GZ_TILE;
@@ -1302,19 +1387,14 @@ __global__ void __launch_bounds__(GZ_BIG_THREADS) k_gz_big(GapArgs A) {
     for (int tile = t0; tile < t1; tile++) nbig += A.cnt[((int64_t)f * A.ntiles + tile) * 3 + 2];
     if (nbig == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    // groups of nw waves (R above the workgroup's threads loops)
-    const int nw = A.big_nw;
-    const int ngroups = (GZ_BIG_THREADS / 64) / nw;
-    const int group = wv / nw;                       // waves past the last whole group only compact
-    const int rl = (wv - group * nw) * 64 + lane;    // realization within the group's span
-    const int span = nw * 64;
-    for (int rbase = 0; rbase < R; rbase += span) {
-        const int r = rbase + rl;
-        const bool on = group < ngroups && r < R;
+    for (int rbase = 0; rbase < R; rbase += GZ_BIG_THREADS) {
+        const int rb = min(GZ_BIG_THREADS, R - rbase);
+        const bool on = tid < rb;
+        const int r = rbase + tid;
         const int64_t pr = ((int64_t)f * A.nchunks + chunk) * R + r;
         Acc<MODE, LM, NP> acc;
         acc.init();
-        if (on && group == 0) {
+        if (on) {
             acc.tot = A.p_total[pr];
 #pragma unroll
             for (int k = 0; k < NP; k++) acc.pt[k] = (k < A.npar) ? A.p_ptot[(int64_t)k * F * A.nchunks * R + pr] : 0.0;
@@ -1324,99 +1404,57 @@ __global__ void __launch_bounds__(GZ_BIG_THREADS) k_gz_big(GapArgs A) {
                               A.p_bin + o, L, R);
             }
         }
+        const int per_round = min(GZ_BIG_RECS, GZ_BIG_PAIRS / rb);
         for (int tile = t0; tile < t1; tile++) {
             const int64_t ft = (int64_t)f * A.ntiles + tile;
             if (A.cnt[ft * 3 + 2] == 0) continue;
             const int nd = A.cnt[ft * 3];
-            // GZ_BIG_THREADS / 4 dense records at a time: those without a table, in order
-            for (int c = 0; c < nd; c += GZ_BIG_THREADS / 4) {
-                const int i = c + tid;
-                bool big = false;
-                GzBigRec q;
-                if (tid < GZ_BIG_THREADS / 4 && i < nd) {
-                    const DRec d = A.drec[ft * GZ_REC + i];
-                    big = d.n == 0;
+            const DRec* rec = A.drec + ft * GZ_REC;
+            int nl = 0;
+            for (int c = 0; c < nd; c += GZ_BIG_THREADS) {
+                const bool big = c + tid < nd && rec[c + tid].n == 0;
+                const uint64_t mask = __ballot(big);
+                __syncthreads();   // the list and counts of before have been read
+                if (lane == 0) s_cnt[wv] = __popcll(mask);
+                __syncthreads();
+                int off = nl;
+                for (int w = 0; w < GZ_BIG_WAVES; w++) {
+                    if (w < wv) off += s_cnt[w];
+                    nl += s_cnt[w];
+                }
+                if (big) s_list[off + gz_below(mask, lane)] = (uint16_t)(c + tid);
+            }
+            for (int c = 0; c < nl; c += per_round) {
+                const int nr = min(per_round, nl - c);
+                __syncthreads();   // the list is whole; the last round has been added up
+                if (tid < nr) {
+                    GzBigRec q;
+                    q.i = s_list[c + tid];
+                    const DRec d = rec[q.i];
                     q.lam = d.lam;
                     q.h = d.h;
                     q.word = d.word;
-                    q.i = i;
-                }
-                const uint64_t mask = __ballot(big);
-                __syncthreads();   // the previous records' readers are done
-                if (lane == 0) s_cnt[wv] = __popcll(mask);
-                __syncthreads();
-                int off = 0, nb = 0;
-                for (int w = 0; w < GZ_BIG_THREADS / 256; w++) {
-                    if (w < wv) off += s_cnt[w];
-                    nb += s_cnt[w];
-                }
-                if (big) {
                     const double slam = sqrt(q.lam);
                     q.loglam = log(q.lam);
                     q.b = 0.931 + 2.53 * slam;
                     q.a = -0.059 + 0.02483 * q.b;
                     q.log_ia = log(1.1239 + 1.1328 / (q.b - 3.4));
                     q.vr = 0.9277 - 3.6224 / (q.b - 2);
-                    s_rec[off + __popcll(mask & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))))] = q;
+                    s_rec[tid] = q;
                 }
                 __syncthreads();
+                gz_big_draw(A, s_rec, s_q[wv], s_n, nr * rb, rb, rbase, f, wv, lane);
+                __syncthreads();
                 if (on)
-                    for (int k = group; k < nb; k += ngroups) {
-                        const GzBigRec& s = s_rec[k];
-                        const uint32_t bin = (uint32_t)(s.word >> 32);
-                        double n;
-                        if (s.lam > A.thresh || s.lam < 10.0) {
-                            n = gz_fallback(bin, (uint32_t)f, (uint32_t)r, 3u, A.seed, s.lam, A.thresh);
-                        } else {
-                            Stream st;
-                            st.init(bin, (uint32_t)f, (uint32_t)r, 3u, A.seed);
-                            n = gz_ptrs(st, s);
-                        }
-                        acc.add(n, s.h, s.word, A.d_par + ft * GZ_TILE + s.i, pstride, A.npar, L);
-                        if (REC) gz_record(A, s.word, f, r, n, false);
+                    for (int j = 0; j < nr; j++) {
+                        const GzBigRec& q = s_rec[j];
+                        const double n = s_n[j * rb + tid];
+                        acc.add(n, q.h, q.word, A.d_par + ft * GZ_TILE + q.i, pstride, A.npar, L);
+                        if (REC) gz_record(A, q.word, f, r, n, false);
                     }
             }
         }
-        // the groups' partials, one group at a time in order, into group 0's
-        for (int g = 1; g < ngroups; g++) {
-            double* s_tot = gz_big_lds;                       // span
-            double* s_pt = s_tot + span;                      // npar x span
-            uint64_t* s_key = (uint64_t*)(s_pt + (int64_t)A.npar * span);   // L x span: (bin << 32 | rank) word
-            __syncthreads();
-            if (group == g) {
-                s_tot[rl] = acc.tot;
-#pragma unroll
-                for (int k = 0; k < NP; k++)
-                    if (k < A.npar) s_pt[k * span + rl] = acc.pt[k];
-                if (MODE != HD_SEL_NONE) {
-#pragma unroll
-                    for (int j = 0; j < LM; j++)
-                        if (j < L) {
-                            if constexpr (MODE == HD_SEL_SORTED) ((uint32_t*)s_key)[j * span + rl] = acc.list.k32(j);
-                            else {
-                                s_key[j * span + rl] = acc.list.key_at(j);
-                                ((int32_t*)(s_key + (int64_t)L * span))[j * span + rl] = acc.list.bin_at(j, A.order);
-                            }
-                        }
-                }
-            }
-            __syncthreads();
-            if (on && group == 0) {
-                acc.tot += s_tot[rl];
-#pragma unroll
-                for (int k = 0; k < NP; k++)
-                    if (k < A.npar) acc.pt[k] += s_pt[k * span + rl];
-                if (MODE != HD_SEL_NONE)
-                    for (int j = 0; j < L; j++) {
-                        if constexpr (MODE == HD_SEL_SORTED)
-                            acc.list.merge(((const uint32_t*)s_key)[j * span + rl], L);
-                        else
-                            acc.list.merge(s_key[j * span + rl],
-                                           ((const int32_t*)(s_key + (int64_t)L * span))[j * span + rl], L);
-                    }
-            }
-        }
-        if (on && group == 0) gz_store<MODE, LM, NP>(A, acc, pr);
+        if (on) gz_store<MODE, LM, NP>(A, acc, pr);
     }
 }
 
@@ -1606,18 +1644,7 @@ static int gz_launch_k(const GapArgs& A, dim3 grid, int bs, size_t lds, hipStrea
     }
     int rc = check_launch("k_gz_draw");
     if (rc) return rc;
-    // groups of as few waves as hold the realizations, and LDS for one group's partials; one group of
-    // all waves where R fills them or the partials (many parameters and slots) would pass 48 KB
-    GapArgs Ab = A;
-    Ab.big_nw = (int)std::min((int64_t)GZ_BIG_THREADS / 64, cdiv(A.R, 64));
-    const size_t per = sizeof(double) * (1 + (size_t)A.npar) +
-                       (MODE == HD_SEL_SORTED ? sizeof(uint32_t) : sizeof(uint64_t) + sizeof(int32_t)) * (size_t)A.L;
-    size_t big_lds = per * Ab.big_nw * 64;
-    if (2 * Ab.big_nw > GZ_BIG_THREADS / 64 || big_lds > 48 * 1024) {
-        Ab.big_nw = GZ_BIG_THREADS / 64;
-        big_lds = 0;
-    }
-    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), grid, dim3(GZ_BIG_THREADS), big_lds, st, Ab);
+    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), grid, dim3(GZ_BIG_THREADS), 0, st, A);
     return check_launch("k_gz_big");
 }
 

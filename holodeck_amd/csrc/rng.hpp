@@ -103,27 +103,6 @@ __device__ __forceinline__ double poisson_inversion(double u, double lam, double
     return n;
 }
 
-// PTRS transformed rejection (W. Hoermann, "The transformed rejection method
-// for generating Poisson random variables", Insurance: Mathematics and
-// Economics 12, 1993), for lam >= 10.
-__device__ __forceinline__ double poisson_ptrs(Stream& st, double lam) {
-    double slam = sqrt(lam), loglam = log(lam);
-    double b = 0.931 + 2.53 * slam;
-    double a = -0.059 + 0.02483 * b;
-    double invalpha = 1.1239 + 1.1328 / (b - 3.4);
-    double vr = 0.9277 - 3.6224 / (b - 2);
-    for (int it = 0; it < 100000; it++) {
-        double U = st.next() - 0.5;
-        double V = st.next();
-        double us = 0.5 - fabs(U);
-        double k = floor((2 * a / us + b) * U + lam + 0.43);
-        if ((us >= 0.07) && (V <= vr)) return k;
-        if ((k < 0) || ((us < 0.013) && (V > us))) continue;
-        if ((log(V) + log(invalpha) - log(a / (us * us) + b)) <= (-lam + k * loglam - lgamma(k + 1.0))) return k;
-    }
-    return floor(lam);   // unreachable in practice; keeps the loop bounded
-}
-
 // Normal(lam, sqrt(lam)) by Box-Muller, not floored (cyutils.pyx:1328-1332).
 __device__ __forceinline__ double normal_count(Stream& st, double lam) {
     double u1 = st.next(), u2 = st.next();
