@@ -85,23 +85,27 @@ constexpr double GZ_CENTRE = 4.0;                 // half-width of a table in st
 
 // dense record (and the sparse pseudo-record at index nd)
 struct DRec {
-    double lam, h;
+    // what a draw needs (GzDraw, one scalar load), then what only the build needs
+    double h;
     uint64_t word;    // bin << 32 | rank
-    double p0;        // Poisson pmf at kb
-    int32_t kb;       // first count of the support (klo): the table build starts here
     int32_t n;        // table length (0: no table, use the fallback sampler)
     int32_t off;      // offset of the table in the tile's concatenated tables
     int32_t kt;       // count of the table's first entry
+    int32_t kb;       // first count of the support (klo): the table build starts here
+    double lam;
+    double p0;        // Poisson pmf at kb
 };
 
-// header of a record staged in LDS for the draw loop (off relative to the batch's table)
+// header of a record staged in LDS for the builds and the tail walks (off relative to the batch's table)
 struct BRec {
-    double h;
-    uint64_t word;
-    double lam;
+    double lam, p0;       // p0: pmf at kb (the build's start)
+    double inv, inv_lo;   // 1 / lam = inv + inv_lo
     int32_t kt, n, off, kb;
-    double p0;   // pmf at kb (the build's start)
 };
+__device__ __forceinline__ BRec gz_header(double lam, double p0, int kt, int n, int off, int kb) {
+    const double inv = 1.0 / lam;
+    return BRec{lam, p0, inv, __fma_rn(-lam, inv, 1.0) * inv, kt, n, off, kb};
+}
 
 struct GapArgs {
     const double* number;   // (B,F)
@@ -542,8 +546,9 @@ struct Acc {
         for (int k = 0; k < (NP > 0 ? NP : 1); k++) pt[k] = 0.0;
     }
     // n instances of a bin with strain h (n as drawn; the sorted walk ignores n < 1)
-    __device__ __forceinline__ void add(double n, double h, uint64_t word, const double* p, int64_t pstride, int npar,
-                                        int L) {
+    // p: the bin's parameters, pstride apart (a constant-space pointer where the bin is wave-uniform)
+    template <class Par>
+    __device__ __forceinline__ void add(double n, double h, uint64_t word, Par p, int64_t pstride, int npar, int L) {
         if (MODE == HD_SEL_SORTED ? !(n >= 1.0) : (n == 0.0)) return;
         tot += n * h;
 #pragma unroll
@@ -556,26 +561,17 @@ struct Acc {
     }
 };
 
-// 1/x for x >= 1: hardware reciprocal refined by two Newton steps (about an
-// ulp, against ~10 instructions for the correctly rounded divide).
-__device__ __forceinline__ double gz_rcp(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
-}
-
-// CDF value c in [0, 1] as a 64-bit fixed-point fraction floor(c 2^64) split
-// into its high and low 32-bit words (c >= 1 saturates); exact.
+// CDF value c in [0, 1) as a 64-bit fixed-point fraction, the multiple of 2^-64 nearest to it (exact
+// from 2^-12 on), split into its high and low 32-bit words.  c is below 1 (the callers limit it).
+// The words are taken from the significands of sums with a power of two (full-rate adds; the
+// conversions between doubles and integers run at a quarter of the rate): t holds c 2^32 to the
+// nearest integer, t2 what is left, which borrows from the high word where it is negative.
 __device__ __forceinline__ void gz_fixed64(double c, uint32_t& h, uint32_t& l) {
-    if (!(c < 1.0)) {
-        h = l = 0xFFFFFFFFu;
-        return;
-    }
-    const double t = c * 4294967296.0;   // exact
-    h = (uint32_t)t;
-    l = (uint32_t)((t - (double)h) * 4294967296.0);   // the fraction is exact, so is its scaling
+    const double t = __fma_rn(c, 0x1p32, 0x1p52);
+    const double d = __fma_rn(c, 0x1p32, 0x1p52 - t);           // exact
+    const double t2 = __fma_rn(d, 0x1p32, 0x1.8p52);
+    h = (uint32_t)__double2loint(t) + (uint32_t)((__double2hiint(t2) - 0x43380000) >> 31);
+    l = (uint32_t)__double2loint(t2);
 }
 
 // Inclusive scans of doubles over groups of G lanes (G = 16: each DPP row; G = 64:
@@ -616,144 +612,152 @@ struct GzMax { __device__ double operator()(double a, double b) const { return f
 
 // Build the CDF table of a record with a group of G lanes (G = 16: four records
 // per wave, one per DPP row; G = 64: one record per wave), as 64-bit fixed point:
-// hi[0, n) the high words, hi[n, 2n) the low words, entry j = floor(2^64 CDF(kt + j))
+// hi[0, n) the high words, hi[n, 2n) the low words, entry j = CDF(kt + j) 2^64
 // with the CDF summed from kb.  The counts kb .. kt + n - 1 are split into
-// contiguous segments of the group's lanes; p(kb) = p0 comes from the prep kernel
-// and the pmf follows p(k+1) = p(k) lam / (k+1).  Pass 1: each lane's pmf relative
-// to its segment's first count, their product and their sum (the running relative
-// sums at the table's counts parked in the table's own words); a group prefix
-// product gives each segment's first pmf, a group prefix sum of the segment sums
-// the carries.  Pass 2 writes carry + first pmf * relative sum (one rounding, fma)
-// for the counts from kt on (lanes wholly below kt write nothing: the lower tail is
-// only summed).  (Relative error of the CDF about
-// (kt + n - kb) ulp, then rounding down to a multiple of 2^-64.)  Four records per
-// wave share the fixed cost of the scans; long tables take a whole wave, which
-// shortens each lane's serial recurrence (the builds of a batch are its critical
-// path).  Arguments are the group's record (n = 0 and kt = kb: no table, the group
-// idles); gl = lane index within the group; the whole wave calls (the scans read
-// every lane).
+// contiguous segments of the group's lanes; p(kb) = p0 comes from the prep kernel.
+// Within a segment the pmf runs downwards from its last count, p(k-1) = p(k) k / lam: two
+// multiplications and the correction of 1 / lam's rounding, where upwards every count takes a
+// reciprocal (a quarter-rate instruction and four more).  Pass 1: each lane's pmf relative to its
+// segment's last count, summed from there (the sum above a count parked in the table's own words);
+// one reciprocal per lane and a group prefix product give each segment's last pmf, a group prefix
+// sum of the segment sums the carries.  Pass 2 writes carry + last pmf * (segment sum - parked sum)
+// (one rounding, fma) for the counts from kt on (lanes wholly below kt write nothing: the lower
+// tail is only summed).  The carries round independently of the segment sums, so neighbouring
+// segments could meet out of order by an ulp: the carries are made non-decreasing (a prefix
+// maximum) and a segment's entries are limited by the next one's carry, so the table is exactly
+// non-decreasing and the inversion a monotone map of the uniform.  (Relative error of the CDF about
+// (kt + n - kb) ulp, then the nearest multiple of 2^-64.)  Four records per wave share the fixed cost
+// of the scans; long tables take a whole wave, which shortens each lane's serial recurrence (the builds
+// of a batch are its critical path).  A segment's length is odd: the lanes' entries, that many words
+// apart, then fall into different LDS banks.  Arguments are the group's record (on = false: no table,
+// the group idles); gl = lane index within the group; the whole wave calls (the scans read every lane).
 typedef __attribute__((address_space(3))) uint32_t gz_lds_u32;
+typedef const __attribute__((address_space(3))) BRec* gz_lrec;
+
+// 1/x for normal x: hardware reciprocal refined by two Newton steps (about an ulp)
+__device__ __forceinline__ double gz_rcp(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    double e = __fma_rn(-x, r, 1.0);
+    r = __fma_rn(e, r, r);
+    e = __fma_rn(-x, r, 1.0);
+    return __fma_rn(e, r, r);
+}
+
+// Pass 1 of one lane: the m counts from j0 on (of those from kb on); jt = the lane's index of the
+// table's first count.  sum: of the segment's pmf relative to its last count; up: its last pmf over
+// the previous count's (from_first: over its own first count's; 1 without counts).
+__device__ __forceinline__ void gz_segment(gz_lds_u32* hi, gz_lds_u32* lo, double inv, double inv_lo, int kb, int j0,
+                                           int m, int jt, bool from_first, double& sum, double& up) {
+    double k = (double)(kb + j0 + m - 1), q = 1.0;
+    sum = 0.0;
+    int j = m - 1;
+    const int jp = max(jt, 1);
+    gz_lds_u32* ph = hi + (j - jt);
+    gz_lds_u32* pl = lo + (j - jt);
+#pragma unroll 4
+    for (; j >= jp; j--) {   // counts of the table
+        *ph-- = (uint32_t)__double2loint(sum);
+        *pl-- = (uint32_t)__double2hiint(sum);
+        sum += q;
+        q *= __fma_rn(k, inv_lo, k * inv);
+        k -= 1.0;
+    }
+#pragma unroll 4
+    for (; j > 0; j--) {     // counts below it
+        sum += q;
+        q *= __fma_rn(k, inv_lo, k * inv);
+        k -= 1.0;
+    }
+    if (m > 0) {
+        if (jt <= 0) {
+            hi[-jt] = (uint32_t)__double2loint(sum);
+            lo[-jt] = (uint32_t)__double2hiint(sum);
+        }
+        sum += q;
+    }
+    if (!from_first) q *= __fma_rn(k, inv_lo, k * inv);
+    up = (m > 0) ? gz_rcp(q) : 1.0;
+}
+
+// Pass 2 of one lane: entries carry + plast * (sum - parked sum), at most `most`
+__device__ __forceinline__ void gz_entries(gz_lds_u32* hi, gz_lds_u32* lo, int m, int jt, double plast, double sum,
+                                           double carry, double most) {
+    most = __builtin_fmin(most, 1.0 - 0x1p-53);
+    const int j0 = max(jt, 0);
+    gz_lds_u32* ph = hi + (j0 - jt);
+    gz_lds_u32* pl = lo + (j0 - jt);
+#pragma unroll 4
+    for (int j = j0; j < m; j++) {
+        const double r = sum - __hiloint2double((int)*pl, (int)*ph);
+        uint32_t h, l;
+        gz_fixed64(__builtin_fmin(__fma_rn(plast, r, carry), most), h, l);
+        *ph++ = h;
+        *pl++ = l;
+    }
+}
+
 template <int G>
-__device__ __noinline__ void gz_build(gz_lds_u32* hi, double lam, int kb, int kt, int n, double p0, int gl) {
+__device__ __noinline__ void gz_build(gz_lrec rec, gz_lds_u32* hi, bool on, int gl) {
+    const int n = on ? rec->n : 0, kb = rec->kb, kt = on ? rec->kt : kb;
     gz_lds_u32* lo = hi + n;
     const int nb = kt + n - kb;          // counts summed
-    const int s = (nb + G - 1) / G;
+    const int s = ((nb + G - 1) / G) | 1;
     const int j0 = gl * s;
     const int m = min(max(nb - j0, 0), s);
-    const double kf = (double)(kb + j0);
     const int jt = kt - kb - j0;         // segment index of the table's first count
-    // pass 1; the relative sum at every count of the table is parked in that entry's own two
-    // words (low half in the high-word slot, high half in the low-word slot) for pass 2
-    double prod = 1.0, rel = 0.0;
-    for (int j = 0; j < m; j++) {
-        rel += prod;
-        if (j >= jt) {
-            hi[j0 + j - (kt - kb)] = (uint32_t)__double2loint(rel);
-            lo[j0 + j - (kt - kb)] = (uint32_t)__double2hiint(rel);
-        }
-        prod *= lam * gz_rcp(kf + (double)(j + 1));
-    }
-    const double pre = gz_group_prev<G>(gz_group_scan<G>(prod, 1.0, GzMul()), 1.0);   // over the lanes before
-    const double pstart = p0 * pre;      // p(kb + j0)
-    const double local = pstart * rel;
-    const double carry = gz_group_prev<G>(gz_group_scan<G>(local, 0.0, GzAdd()), 0.0);   // sum of those before
-    const double last = (m > 0) ? __fma_rn(pstart, rel, carry) : -1.0;
-    // The carries are rounded independently of the segment sums, so two
-    // neighbouring segments can meet out of order by an ulp; raise each
-    // segment to the largest value before it, which makes the table exactly
-    // non-decreasing (so the inversion is a monotone map of the uniform).
-    const double ninf = -__builtin_inf();
-    const double before = gz_group_prev<G>(gz_group_scan<G>(last, ninf, GzMax()), ninf);
-    // pass 2, for the counts of the table: the parked relative sums (each lane reads back only
-    // what it wrote) and the same fma, so a segment's last value is exactly `last`
-    for (int j = max(jt, 0); j < m; j++) {
-        const int e = j0 + j - (kt - kb);
-        const double r = __hiloint2double((int)lo[e], (int)hi[e]);
-        uint32_t h, l;
-        gz_fixed64(fmax(__fma_rn(pstart, r, carry), before), h, l);
-        hi[e] = h;
-        lo[e] = l;
-    }
+    // pass 1; the sum above every count of the table is parked in that entry's own two words (low
+    // half in the high-word slot, high half in the low-word slot) for pass 2
+    double sum, up;
+    gz_segment(hi, lo, rec->inv, rec->inv_lo, kb, j0, m, jt, gl == 0, sum, up);
+    const double plast = rec->p0 * gz_group_scan<G>(up, 1.0, GzMul());    // pmf of the segment's last count
+    const double upto = gz_group_scan<G>(gz_group_scan<G>(plast * sum, 0.0, GzAdd()), 0.0, GzMax());   // and CDF
+    // pass 2, for the counts of the table (each lane reads back only what it wrote)
+    gz_entries(hi, lo, m, jt, plast, sum, gz_group_prev<G>(upto, 0.0), upto);
 }
 
 // One part of a long table, built by a wave: the counts [j_lo, j_hi) of the kb .. kt + n - 1 summed.
 // Where a batch holds fewer long tables than the workgroup has waves, each is cut into parts so
 // that every wave has one: a lane's serial recurrence, which the whole batch waits for, is then a
-// part's length / 64 instead of the table's.  The part's first pmf comes from the saddle-point form
-// (its own anchor: no product over the earlier parts).  gz_part_sum leaves the part's last running sum in
-// s_part as (first pmf of its last lane, that lane's relative sum, the carry into that lane);
-// gz_part_base of every later part sums these up, and leaves the part's largest value in s_part[3],
-// which the later parts' entries are raised to where rounding would put them below it (as gz_build
-// does between lanes), so the table is non-decreasing; gz_part_write then writes the entries.
+// part's length / 64 instead of the table's.  gz_part_sum does pass 1 relative to the pmf before the
+// part (p0 for the first part) and leaves in s_part the part's pmf ratio, last count to that one, and its
+// sum; after a barrier gz_part_write takes the scale and the CDF before the part from the parts before.
+// (Anchoring each part by its own saddle-point pmf, exchanging the parts' largest values over another
+// barrier and an even segment length, whose LDS accesses met in few banks, made the launch of the
+// eccentric realizations, with tables of 870 entries on average, 32.0 ms: 23.3 now.)
 struct GzPart {
-    double pstart, carry, before;
-    int j0, m;       // this lane's counts
+    double plast, sum, upto;   // relative to the pmf before the part
+    int j0, m;                 // this lane's counts
 };
 
-__device__ __noinline__ GzPart gz_part_sum(gz_lds_u32* hi, double lam, int kb, int kt, int n, double p0, int j_lo,
-                                           int j_hi, int lane, double* s_part) {
-    gz_lds_u32* lo = hi + n;
-    const int nb = j_hi - j_lo;
-    const int s = (nb + 63) >> 6;
+__device__ __noinline__ GzPart gz_part_sum(gz_lrec rec, gz_lds_u32* hi, int j_lo, int j_hi, int lane,
+                                           double* s_part) {
+    const int s = ((j_hi - j_lo + 63) >> 6) | 1;   // odd, as in gz_build
     GzPart P;
     P.j0 = j_lo + lane * s;
     P.m = min(max(j_hi - P.j0, 0), s);
-    const double kf = (double)(kb + P.j0);
-    const int jt = kt - kb - P.j0;
-    const double anchor = (j_lo == 0) ? p0 : gz_pmf_acc(lam, (double)(kb + j_lo));
-    double prod = 1.0, rel = 0.0;
-#pragma unroll 4
-    for (int j = 0; j < P.m; j++) {
-        rel += prod;
-        if (j >= jt) {
-            hi[j - jt] = (uint32_t)__double2loint(rel);
-            lo[j - jt] = (uint32_t)__double2hiint(rel);
-        }
-        prod *= lam * gz_rcp(kf + (double)(j + 1));
-    }
-    P.pstart = anchor * gz_group_prev<64>(gz_group_scan<64>(prod, 1.0, GzMul()), 1.0);
-    P.carry = gz_group_prev<64>(gz_group_scan<64>(P.pstart * rel, 0.0, GzAdd()), 0.0);
-    if (P.m > 0 && P.j0 + P.m == j_hi) {   // the lane of the part's last count
-        s_part[0] = P.pstart;
-        s_part[1] = rel;
-        s_part[2] = P.carry;
+    double up;
+    gz_segment(hi, hi + rec->n, rec->inv, rec->inv_lo, rec->kb, P.j0, P.m, rec->kt - rec->kb - P.j0,
+               j_lo == 0 && lane == 0, P.sum, up);
+    P.plast = gz_group_scan<64>(up, 1.0, GzMul());
+    P.upto = gz_group_scan<64>(gz_group_scan<64>(P.plast * P.sum, 0.0, GzAdd()), 0.0, GzMax());
+    if (lane == 63) {
+        s_part[0] = P.plast;   // lanes without counts have up = 1: the part's last count
+        s_part[1] = P.upto;
     }
     return P;
 }
 
-// part: its index; s_part: the part sums of the table's part 0 (4 doubles each)
-__device__ __noinline__ void gz_part_base(gz_lds_u32* hi, int kb, int kt, int n, GzPart& P, int part, int lane,
-                                          double* s_part) {
-    const gz_lds_u32* lo = hi + n;
-    const int jt = kt - kb - P.j0;
-    double base = 0.0;
-    for (int q = 0; q < part; q++) base = __fma_rn(s_part[4 * q], s_part[4 * q + 1], base + s_part[4 * q + 2]);
-    P.carry += base;
-    // the lane's last value (the parked relative sum; none below the table)
-    const int e = P.m - 1 - jt;
-    const double ninf = -__builtin_inf();
-    double last = ninf;
-    if (P.m > 0 && e >= 0) last = __fma_rn(P.pstart, __hiloint2double((int)lo[e], (int)hi[e]), P.carry);
-    const double upto = gz_group_scan<64>(last, ninf, GzMax());
-    P.before = gz_group_prev<64>(upto, ninf);
-    if (lane == 63) s_part[4 * part + 3] = upto;
-}
-
-__device__ __noinline__ void gz_part_write(gz_lds_u32* hi, int kb, int kt, int n, GzPart P, int part,
+// part: its index; s_part: the sums of the table's part 0 (2 doubles each)
+__device__ __noinline__ void gz_part_write(gz_lrec rec, gz_lds_u32* hi, GzPart P, int part,
                                            const double* s_part) {
-    gz_lds_u32* lo = hi + n;
-    const int jt = kt - kb - P.j0;
-    double before = P.before;
-    for (int q = 0; q < part; q++) before = fmax(before, s_part[4 * q + 3]);
-#pragma unroll 4
-    for (int j = max(jt, 0); j < P.m; j++) {
-        const int e = j - jt;
-        const double r = __hiloint2double((int)lo[e], (int)hi[e]);
-        uint32_t h, l;
-        gz_fixed64(fmax(__fma_rn(P.pstart, r, P.carry), before), h, l);
-        hi[e] = h;
-        lo[e] = l;
+    double scale = rec->p0, base = 0.0;
+    for (int q = 0; q < part; q++) {
+        base = __fma_rn(scale, s_part[2 * q + 1], base);
+        scale *= s_part[2 * q];
     }
+    const double upto = __fma_rn(scale, P.upto, base);   // non-decreasing over lanes and parts
+    const double carry = gz_group_prev<64>(upto, base);
+    gz_entries(hi, hi + rec->n, P.m, rec->kt - rec->kb - P.j0, scale * P.plast, P.sum, carry, upto);
 }
 
 // Parts of each of nl long tables for a workgroup of GZ_WAVES waves; below GZ_SPLIT_MIN counts
@@ -774,29 +778,34 @@ __device__ __forceinline__ int gz_part_edge(int nb, int part, int parts) { retur
 #endif
 
 // A short table built by one thread in one pass: the same entries as gz_build
-// (the CDF summed from kb by the pmf recurrence, floor(2^64 CDF) as high and low
-// words), the sum running in order, so the entries are non-decreasing as they
-// are.  For tables whose counts kb .. kt + n - 1 number at most GZ_SEQ_MAX: a
-// thread per table avoids the wave scans, which cost more than such a table.
+// (the CDF summed from count 0 by the pmf recurrence), the sum running in order, so the
+// entries are non-decreasing as they are.  For tables whose counts number at most GZ_SEQ_MAX: a
+// thread per table avoids the wave scans, which cost more than such a table.  Such a table starts
+// at count 0 (a support that starts above 0 has lam > 77 and more counts), so the count is the same
+// in every lane and its reciprocal a scalar load.
 #ifndef HD_GZ_SEQ_MAX
 #define HD_GZ_SEQ_MAX 32
 #endif
 constexpr int GZ_SEQ_MAX = HD_GZ_SEQ_MAX;
-__device__ __forceinline__ void gz_build_seq(uint32_t* hi, double lam, int kb, int kt, int n, double p0) {
-    uint32_t* lo = hi + n;
+static_assert(GZ_SEQ_MAX <= 32, "reciprocals of the counts of a short table");
+__constant__ double gz_inv_k[33] = {
+    0.0, 1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5, 1.0 / 6, 1.0 / 7, 1.0 / 8, 1.0 / 9, 1.0 / 10, 1.0 / 11, 1.0 / 12,
+    1.0 / 13, 1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17, 1.0 / 18, 1.0 / 19, 1.0 / 20, 1.0 / 21, 1.0 / 22, 1.0 / 23,
+    1.0 / 24, 1.0 / 25, 1.0 / 26, 1.0 / 27, 1.0 / 28, 1.0 / 29, 1.0 / 30, 1.0 / 31, 1.0 / 32};
+__device__ __forceinline__ void gz_build_seq(gz_lds_u32* hi, double lam, int kt, int n, double p0) {
+    gz_lds_u32* lo = hi + n;
     double p = p0, c = 0.0;
-    int k = kb;
-    for (; k < kt; k++) {   // the lower tail, summed into entry 0
+    const int nb = kt + n;
+    for (int k = 0; k < GZ_SEQ_MAX; k++) {   // the counts below kt are summed into entry 0
+        if (k >= nb) break;
         c += p;
-        p *= lam * gz_rcp((double)(k + 1));
-    }
-    for (int j = 0; j < n; j++, k++) {
-        c += p;
-        uint32_t h, l;
-        gz_fixed64(c, h, l);
-        hi[j] = h;
-        lo[j] = l;
-        p *= lam * gz_rcp((double)(k + 1));
+        if (k >= kt) {
+            uint32_t h, l;
+            gz_fixed64(__builtin_fmin(c, 1.0 - 0x1p-53), h, l);
+            hi[k - kt] = h;
+            lo[k - kt] = l;
+        }
+        p *= lam * gz_inv_k[k + 1];
     }
 }
 
@@ -934,13 +943,25 @@ __device__ __forceinline__ int gz_draw1(const GzTab& t, Words& rs) {
     return gz_count(t, j, x, w, hw, rs);
 }
 
+// The candidate of a finished search: count kt + j, and whether it stands as it is -- no tie on the high
+// word (the low words decide) and j within the table (j in [lo, n), lo = 1 when entry 0 carries a
+// summed lower tail).
+__device__ __forceinline__ int gz_candidate(const GzTab& t, const gz_lds_u32* p, uint32_t x, bool& stands) {
+    const uint32_t h0 = p[0], h1 = p[1];
+    const bool up = h0 < x;
+    const int j = gz_idx(p, t.hi) + (up ? 1 : 0);
+    const int lo = (t.kt > t.kb) ? 1 : 0;
+    stands = ((uint32_t)(j - lo) < (uint32_t)(t.n - lo)) & ((up ? h1 : h0) != x);
+    return t.kt + j;
+}
+
 // Two draws from tables a and b (n = 0: no draw, count 0).  Words in the order
 // x_a, x_b, then w_a, w_b where a tie needs them, then w_a, w_b where a tail
 // walk needs them and the search did not take them.
-
 template <class Words>
 __device__ __forceinline__ void gz_draw2(const GzTab& ta, const GzTab& tb, Words& rs, int& ca, int& cb) {
     GzSearch a, b;
+    const bool both = ta.n > 0 && tb.n > 0;   // uniform, and nearly always so
     const uint32_t xa = (ta.n > 0) ? rs.next() : 0u;
     const uint32_t xb = (tb.n > 0) ? rs.next() : 0u;
     gz_search_start(a, ta.hi, ta.n, xa);
@@ -959,20 +980,13 @@ __device__ __forceinline__ void gz_draw2(const GzTab& ta, const GzTab& tb, Words
     }
     while (a.len > 1) gz_search_step(a);
     while (b.len > 1) gz_search_step(b);
-    {   // the common case: no lane of the wave has a tie on a high word (the low words needed)
-        // or a draw outside a table, so every count is kt + j from the candidates alone (one
-        // wave-wide test instead of per-lane branches); otherwise the exact path below
-        const uint32_t a0 = a.p[0], a1 = a.p[1], b0 = b.p[0], b1 = b.p[1];
-        const bool ua = a0 < xa, ub = b0 < xb;
-        const int ja = gz_idx(a.p, a.hi) + (ua ? 1 : 0), jb = gz_idx(b.p, b.hi) + (ub ? 1 : 0);
-        // fast: no tie on a high word and j in [lo, n) (lo = 1 when entry 0 carries a summed lower
-        // tail), as in gz_draw1; straight-line code on masks
-        const int loa = (ta.kt > ta.kb) ? 1 : 0, lob = (tb.kt > tb.kb) ? 1 : 0;
-        const bool fa = ((uint32_t)(ja - loa) < (uint32_t)(ta.n - loa)) & ((ua ? a1 : a0) != xa);
-        const bool fb = ((uint32_t)(jb - lob) < (uint32_t)(tb.n - lob)) & ((ub ? b1 : b0) != xb);
-        if (__builtin_amdgcn_ballot_w64(((ta.n > 0) & !fa) | ((tb.n > 0) & !fb)) == 0ull) {
-            ca = (ta.n > 0) ? ta.kt + ja : 0;
-            cb = (tb.n > 0) ? tb.kt + jb : 0;
+    if (both) {   // the common case: every lane's two candidates stand (one wave-wide test instead of
+                  // per-lane branches); otherwise the exact path below
+        bool fa, fb;
+        const int ka = gz_candidate(ta, a.p, xa, fa), kb = gz_candidate(tb, b.p, xb, fb);
+        if (__builtin_amdgcn_ballot_w64(!(fa & fb)) == 0ull) {
+            ca = ka;
+            cb = kb;
             return;
         }
     }
@@ -996,22 +1010,29 @@ __device__ __forceinline__ GzTab gz_tab(const uint32_t* tab, const BRec* b, bool
     return t;
 }
 
-// The table of a record read from global memory through the constant address space (the
-// fields are wave-uniform: scalar loads); off is relative to the batch's first table.
-typedef const __attribute__((address_space(4))) DRec* gz_cdrec;
-__device__ __forceinline__ DRec gz_load_rec(gz_cdrec p) {
-    DRec d;
-    d.lam = p->lam;
-    d.h = p->h;
-    d.word = p->word;
-    d.p0 = p->p0;
-    d.kb = p->kb;
-    d.n = p->n;
-    d.off = p->off;
-    d.kt = p->kt;
+// The draw part of a record read from global memory through the constant address space: wave-uniform,
+// one scalar load of eight words.
+struct GzDraw {
+    double h;
+    uint64_t word;
+    int n, off, kt, kb;
+};
+typedef uint32_t gz_u32x8 __attribute__((ext_vector_type(8)));
+typedef const __attribute__((address_space(4))) gz_u32x8* gz_cdraw;
+typedef const __attribute__((address_space(4))) double* gz_cpar;
+static_assert(sizeof(DRec) == 48, "a record's draw part is its first 32 bytes");
+__device__ __forceinline__ GzDraw gz_load_draw(const DRec* rec) {
+    const gz_u32x8 w = *(gz_cdraw)rec;
+    GzDraw d;
+    d.h = __hiloint2double((int)w[1], (int)w[0]);
+    d.word = ((uint64_t)w[3] << 32) | w[2];
+    d.n = (int)w[4];
+    d.off = (int)w[5];
+    d.kt = (int)w[6];
+    d.kb = (int)w[7];
     return d;
 }
-__device__ __forceinline__ GzTab gz_tab_rec(const uint32_t* tab, const DRec& d, int base, const BRec* staged,
+__device__ __forceinline__ GzTab gz_tab_rec(const uint32_t* tab, const GzDraw& d, int base, const BRec* staged,
                                             bool present) {
     GzTab t;
     t.n = present ? d.n : 0;
@@ -1055,7 +1076,8 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     __shared__ int s_nrow;             // mid-size tables (a 16-lane row each)
     __shared__ int s_nshort;           // short tables (a lane each)
     __shared__ int s_lsum;             // counts summed over the long tables
-    __shared__ double s_part[GZ_WAVES][4];   // sums of the parts of split long tables
+    __shared__ double s_part[GZ_WAVES][2];   // ratios and sums of the parts of split long tables
+    __shared__ int s_cnt[GZ_TPC_MAX][2];     // dense and sparse counts of the item's tiles
     __shared__ int s_large[GZ_BATCH_REC];
     __shared__ int s_row[GZ_BATCH_REC];
     __shared__ int s_short[GZ_BATCH_REC];
@@ -1072,6 +1094,12 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     const int t1 = min(t0 + A.tpc, A.ntiles);
     const int64_t pstride = (int64_t)F * A.ntiles * GZ_TILE;
     const uint32_t k0 = (uint32_t)A.seed, k1 = (uint32_t)(A.seed >> 32);
+    if (tid < t1 - t0) {
+        const int32_t* cnt = A.cnt + ((int64_t)f * A.ntiles + t0 + tid) * 3;
+        s_cnt[tid][0] = cnt[0];
+        s_cnt[tid][1] = cnt[1];
+    }
+    __syncthreads();
 
     for (int rbase = 0; rbase < R; rbase += bs) {
         const int r = rbase + tid;
@@ -1082,28 +1110,26 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
             const int64_t ft = (int64_t)f * A.ntiles + tile;
             const int64_t reg = ft * GZ_TILE;
             const int64_t rreg = ft * GZ_REC;
-            const int nd = A.cnt[ft * 3];
-            const int ns = A.cnt[ft * 3 + 1];
+            const int nd = s_cnt[tile - t0][0], ns = s_cnt[tile - t0][1];
             const int nrec = nd + (ns > 0 ? 1 : 0);
             // the realization's stream for this tile: records in order take one word each
             // (two when the 32-bit draw is open), then the sparse points two words each
             Xo128 rs;
             rs.seed(philox4x32_10(U4{(uint32_t)tile, (uint32_t)f, (uint32_t)r, 6u << 16}, k0, k1));
-            int c = 0;
+            int c = 0, base = 0;   // base: where the batch's tables start among the tile's
             while (c < nrec) {
-                // batch [c, c1): consecutive records whose windows fit the table
-                const int base = (c == 0) ? 0 : A.rec_end[rreg + c - 1];
+                // batch [c, c1): consecutive records whose windows fit the table, at most
+                // GZ_BATCH_REC.  The record this thread stages is loaded with the record ends: its
+                // place does not depend on where the batch ends
+                const DRec mine = A.drec[rreg + min(c + tid, nrec - 1)];
+                const int e0 = A.rec_end[rreg + min(c + lane, nrec - 1)];
+                const int e1 = A.rec_end[rreg + min(c + 64 + lane, nrec - 1)];
                 const int limit = base + A.cap;
-                int c1 = c;
-                for (;;) {
-                    const int idx = c1 + lane;
-                    const int e = (idx < nrec) ? A.rec_end[rreg + idx] : 0x7fffffff;
-                    const int adv = __popcll(__ballot(e <= limit));
-                    c1 += adv;
-                    if (adv < 64) break;
-                }
+                int c1 = c + __popcll(__ballot(c + lane < nrec && e0 <= limit)) +
+                         __popcll(__ballot(c + 64 + lane < nrec && e1 <= limit));
                 c1 = max(c1, c + 1);   // every window fits alone (n <= cap); keeps progress unconditional
-                c1 = min(c1, c + GZ_BATCH_REC);
+                const int base_next = (c1 - c <= 64) ? __builtin_amdgcn_readlane(e0, c1 - c - 1)
+                                                     : __builtin_amdgcn_readlane(e1, c1 - c - 65);
                 if (tid == 0) {
                     s_next = 0;
                     s_nlarge = 0;
@@ -1115,8 +1141,8 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                 // one thread per record of the batch stages its header and lists its table as
                 // short (at most GZ_SEQ_MAX counts summed) or long
                 if (c + tid < c1) {
-                    const DRec rec = A.drec[rreg + c + tid];
-                    brec[tid] = BRec{rec.h, rec.word, rec.lam, rec.kt, rec.n, rec.off - base, rec.kb, rec.p0};
+                    const DRec& rec = mine;
+                    brec[tid] = gz_header(rec.lam, rec.p0, rec.kt, rec.n, rec.off - base, rec.kb);
                     const int nb = rec.kt + rec.n - rec.kb;
                     if (rec.n > 0 && nb <= GZ_SEQ_MAX) s_short[atomicAdd(&s_nshort, 1)] = tid;
                     else if (rec.n > 0 && nb <= HD_GZ_ROW_MAX) s_row[atomicAdd(&s_nrow, 1)] = tid;
@@ -1140,18 +1166,12 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                         const int part = wv % parts, nb = rec->kt + rec->n - rec->kb;
                         const bool on = wv < nl * parts;
                         GzPart P;
+                        gz_lds_u32* hi = (gz_lds_u32*)(tab + 2 * rec->off);
                         if (on)
-                            P = gz_part_sum((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kb, rec->kt, rec->n,
-                                            rec->p0, gz_part_edge(nb, part, parts), gz_part_edge(nb, part + 1, parts),
+                            P = gz_part_sum((gz_lrec)rec, hi, gz_part_edge(nb, part, parts), gz_part_edge(nb, part + 1, parts),
                                             lane, s_part[wv]);
                         __syncthreads();
-                        if (on)
-                            gz_part_base((gz_lds_u32*)(tab + 2 * rec->off), rec->kb, rec->kt, rec->n, P, part, lane,
-                                         s_part[wv - part]);
-                        __syncthreads();
-                        if (on)
-                            gz_part_write((gz_lds_u32*)(tab + 2 * rec->off), rec->kb, rec->kt, rec->n, P, part,
-                                          s_part[wv - part]);
+                        if (on) gz_part_write((gz_lrec)rec, hi, P, part, s_part[wv - part]);
                         nl = 0;
                     }
                     const int nrg = (nr + 3) >> 2, nsg = (nsh + 63) >> 6;
@@ -1162,19 +1182,17 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                         if (w >= nl + nrg + nsg) break;
                         if (w < nl) {
                             const BRec* rec = brec + s_large[w];
-                            gz_build<64>((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kb, rec->kt, rec->n, rec->p0,
-                                         lane);
+                            gz_build<64>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), true, lane);
                         } else if (w < nl + nrg) {
                             const int k = (w - nl) * 4 + (lane >> 4);
                             const bool on = k < nr;
                             const BRec* rec = brec + s_row[on ? k : 0];
-                            gz_build<16>((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, on ? rec->kb : 0, on ? rec->kt : 0,
-                                         on ? rec->n : 0, rec->p0, lane & 15);
+                            gz_build<16>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), on, lane & 15);
                         } else {
                             const int k = (w - nl - nrg) * 64 + lane;
                             if (k < nsh) {
                                 const BRec* rec = brec + s_short[k];
-                                gz_build_seq(tab + 2 * rec->off, rec->lam, rec->kb, rec->kt, rec->n, rec->p0);
+                                gz_build_seq((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kt, rec->n, rec->p0);
                             }
                         }
                     }
@@ -1189,21 +1207,24 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                     // the records' fields are the same for every lane: read through the constant
                     // address space (scalar loads into SGPRs, no VALU moves); the staged LDS copy
                     // serves the builds and the rare tail walk
-                    const gz_cdrec cdr = (gz_cdrec)(A.drec + rreg);
+                    // the next pair's records are loaded before the current pair is drawn
                     const int cd = min(c1, nd);
-                    for (int i = c; i < cd; i += 2) {
-                        const bool hb = i + 1 < cd;
-                        const DRec ra = gz_load_rec(cdr + i);
-                        const DRec rb = gz_load_rec(cdr + (hb ? i + 1 : i));
-                        const GzTab ta = gz_tab_rec(tab, ra, base, brec + (i - c), true);
-                        const GzTab tb = gz_tab_rec(tab, rb, base, brec + (hb ? i + 1 - c : i - c), hb);
-                        int ka, kb;
-                        gz_draw2(ta, tb, rs, ka, kb);
-                        if (ta.n > 0) acc.add((double)ka, ra.h, ra.word, A.d_par + reg + i, pstride, A.npar, L);
-                        if (tb.n > 0) acc.add((double)kb, rb.h, rb.word, A.d_par + reg + i + 1, pstride, A.npar, L);
-                        if (REC) {
-                            if (ta.n > 0) gz_record(A, ra.word, f, r, (double)ka, false);
-                            if (tb.n > 0) gz_record(A, rb.word, f, r, (double)kb, false);
+                    const DRec* rec = A.drec + rreg;
+                    {
+                        for (int i = c; i < cd; i += 2) {
+                            const bool hb = i + 1 < cd;
+                            const GzDraw ra = gz_load_draw(rec + i), rb = gz_load_draw(rec + (hb ? i + 1 : i));
+                            const GzTab ta = gz_tab_rec(tab, ra, base, brec + (i - c), true);
+                            const GzTab tb = gz_tab_rec(tab, rb, base, brec + (hb ? i + 1 - c : i - c), hb);
+                            int ka, kb;
+                            gz_draw2(ta, tb, rs, ka, kb);
+                            const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
+                            if (ta.n > 0) acc.add((double)ka, ra.h, ra.word, par, pstride, A.npar, L);
+                            if (tb.n > 0) acc.add((double)kb, rb.h, rb.word, par + 1, pstride, A.npar, L);
+                            if (REC) {
+                                if (ta.n > 0) gz_record(A, ra.word, f, r, (double)ka, false);
+                                if (tb.n > 0) gz_record(A, rb.word, f, r, (double)kb, false);
+                            }
                         }
                     }
                     for (int i = max(c, nd); i < c1; i++) {
@@ -1231,6 +1252,7 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                     }
                 }
                 c = c1;
+                base = base_next;
             }
         }
         if (active) gz_store<MODE, LM, NP>(A, acc, ((int64_t)f * A.nchunks + chunk) * R + r);
@@ -1463,7 +1485,8 @@ __global__ void __launch_bounds__(GZ_BIG_THREADS, 3) k_gz_big(GapArgs A) {
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(GZ_MAXBS) k_cdf_table_hook(double lam, int cap, int* kn, uint64_t* cdf_out) {
     extern __shared__ double hook_lds[];
-    __shared__ double s_part[GZ_WAVES][4];
+    __shared__ double s_part[GZ_WAVES][2];
+    __shared__ BRec hdr;
     uint32_t* tab = (uint32_t*)hook_lds;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int kb, kt, n;
@@ -1472,21 +1495,19 @@ __global__ void __launch_bounds__(GZ_MAXBS) k_cdf_table_hook(double lam, int cap
         const int nb = kt + n - kb;
         const double p0 = gz_pmf_acc(lam, (double)kb);
         const int parts = gz_parts(1, nb);
+        if (threadIdx.x == 0) hdr = gz_header(lam, p0, kt, n, 0, kb);
+        __syncthreads();
         if (nb <= GZ_SEQ_MAX) {
-            if (threadIdx.x == 0) gz_build_seq(tab, lam, kb, kt, n, p0);
+            if (threadIdx.x == 0) gz_build_seq((gz_lds_u32*)tab, lam, kt, n, p0);
         } else if (nb <= HD_GZ_ROW_MAX) {   // row 0 builds, rows 1-3 idle
-            const bool on = lane < 16;
-            if (wv == 0)
-                gz_build<16>((gz_lds_u32*)tab, lam, on ? kb : 0, on ? kt : 0, on ? n : 0, p0, lane & 15);
+            if (wv == 0) gz_build<16>((gz_lrec)&hdr, (gz_lds_u32*)tab, lane < 16, lane & 15);
         } else if (parts > 1) {
-            GzPart P = gz_part_sum((gz_lds_u32*)tab, lam, kb, kt, n, p0, gz_part_edge(nb, wv, parts),
-                                   gz_part_edge(nb, wv + 1, parts), lane, s_part[wv]);
+            const GzPart P = gz_part_sum((gz_lrec)&hdr, (gz_lds_u32*)tab, gz_part_edge(nb, wv, parts),
+                                         gz_part_edge(nb, wv + 1, parts), lane, s_part[wv]);
             __syncthreads();
-            gz_part_base((gz_lds_u32*)tab, kb, kt, n, P, wv, lane, s_part[0]);
-            __syncthreads();
-            gz_part_write((gz_lds_u32*)tab, kb, kt, n, P, wv, s_part[0]);
+            gz_part_write((gz_lrec)&hdr, (gz_lds_u32*)tab, P, wv, s_part[0]);
         } else if (wv == 0) {
-            gz_build<64>((gz_lds_u32*)tab, lam, kb, kt, n, p0, lane);
+            gz_build<64>((gz_lrec)&hdr, (gz_lds_u32*)tab, true, lane);
         }
     }
     __syncthreads();
@@ -1512,7 +1533,7 @@ __global__ void __launch_bounds__(256) k_table_draw_hook(const uint32_t* tab, in
     uint32_t* t = (uint32_t*)hook_lds;
     __shared__ BRec hdr;
     for (int j = threadIdx.x; j < 2 * n; j += blockDim.x) t[j] = tab[j];
-    if (threadIdx.x == 0) hdr = BRec{0.0, 0, lam, kt, n, 0, kb, 0.0};
+    if (threadIdx.x == 0) hdr = gz_header(lam, 0.0, kt, n, 0, kb);
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m) return;
@@ -1532,8 +1553,8 @@ __global__ void __launch_bounds__(256) k_table_draw_pair_hook(const uint32_t* ta
     __shared__ BRec hdr[2];
     for (int j = threadIdx.x; j < 2 * n2; j += blockDim.x) t2[j] = tab2[j];
     if (threadIdx.x == 0) {
-        hdr[0] = BRec{0.0, 0, lam, kt, n, 0, kb, 0.0};
-        hdr[1] = BRec{0.0, 0, lam2, kt2, n2, 0, kb2, 0.0};
+        hdr[0] = gz_header(lam, 0.0, kt, n, 0, kb);
+        hdr[1] = gz_header(lam2, 0.0, kt2, n2, 0, kb2);
     }
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1572,6 +1593,7 @@ static int gz_cap(int) { return HD_GZ_CAP; }
 // draw workgroup LDS: table + sparse axis + staged headers (+ the build counter); three must fit a
 // 160 KB CU (with the 64 KB per-workgroup limit of the allocation), and the hook's table as well
 constexpr size_t GZ_DRAW_LDS = (size_t)(HD_GZ_CAP + GZ_TILE) * sizeof(double) + (size_t)GZ_BATCH_REC * sizeof(BRec);
+static_assert(GZ_BATCH_REC == 128, "two record ends per lane");
 static_assert(GZ_DRAW_LDS + 16 <= 65536, "draw workgroup LDS above 64 KB");
 // (the static part: the build counters and the three 128-entry lists of k_gz_draw, rounded up)
 static_assert(3 * (GZ_DRAW_LDS + 2048) <= 160 * 1024, "three draw workgroups no longer share a CU");
