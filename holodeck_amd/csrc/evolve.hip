@@ -437,8 +437,8 @@ __global__ void __launch_bounds__(DBN_THREADS, 5) k_dbn_2pwl(EvoConsts K, const 
     }
     __syncthreads();
     // Only the steps whose bracket can hold a target are walked (sorted targets; 1.61 -> 0.73 ms at
-    // 91x81x101 x 40, with the walks of all steps against 0.1 ms of HBM traffic): one evolution from 10^4 pc to the ISCO spans nine decades of separation, the targets of a PTA less than one and a
-    // half.  Below: a step's fr is its rest-frame frequency over 1 + z >= 1, so steps before the first
+    // 91x81x101 x 40): one evolution from 10^4 pc to the ISCO spans nine decades of separation, the
+    // targets of a PTA less than one and a half.  Below: a step's fr is its rest-frame frequency over 1 + z >= 1, so steps before the first
     // with s_frst[step + 1] >= fo[0] record nothing.  Above: once fl is past the last target (or the
     // time past the age of the universe) it stays there, as times and rest-frame frequencies grow; the
     // margins of 1e-3 and 1e-6 cover the rounding of time_left, at most a few 1e-16 of a total time

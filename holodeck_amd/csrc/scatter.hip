@@ -27,12 +27,16 @@
 namespace hd {
 
 // Slot order: slot t is position t of the level schedule (vertex lidx[t]).
-// Adjacency in slot order, padded to CT_SLOT entries per slot: entry k < CT_SLOT
-// of slot t is at t CT_SLOT + k (neighbour -1 past the degree); the entries of a
+// Adjacency padded to CT_SLOT entries per slot (neighbour N past the degree), in planes: entry
+// k < CT_SLOT of slot t is at ((k / L) N + t) L + k % L, L = CT_PIPE_LANES, so that the lanes of the
+// pipelined sweeps (L per vertex, consecutive slots) read each plane in whole lines (with a slot's
+// entries together each load touched the lines of all its slots: 1.18 -> 1.02 ms); the entries of a
 // vertex with more neighbours continue in an overflow area after the N CT_SLOT
 // padded ones, at slot_ovf[t] .. slot_ovf[t+1] (exclusive prefix of the
 // surplus degrees, made here by one workgroup).
 constexpr int CT_SLOT = 8;
+constexpr int CT_PIPE_LANES = 4;                        // lanes per vertex in the pipelined sweeps (a DPP quad)
+constexpr int CT_PIPE_ENT = CT_SLOT / CT_PIPE_LANES;    // entries per lane: lane k holds k, k + CT_PIPE_LANES, ...
 
 __global__ void __launch_bounds__(1024) k_ct_slots(int N, const int32_t* __restrict__ nptr,
                                                    const int32_t* __restrict__ lidx, int32_t* __restrict__ slot_ovf) {
@@ -60,20 +64,22 @@ __global__ void __launch_bounds__(1024) k_ct_slots(int N, const int32_t* __restr
 
 // Index of adjacency entry k of slot t in the padded layout.
 __device__ __forceinline__ int64_t ct_entry(int64_t N, int t, int k, const int32_t* __restrict__ slot_ovf) {
-    return (k < CT_SLOT) ? (int64_t)t * CT_SLOT + k : N * CT_SLOT + slot_ovf[t] + (k - CT_SLOT);
+    return (k < CT_SLOT) ? ((k / CT_PIPE_LANES) * N + t) * CT_PIPE_LANES + k % CT_PIPE_LANES
+                         : N * CT_SLOT + slot_ovf[t] + (k - CT_SLOT);
 }
 
 // Geometry of every slot: the vertex record {p, overflow begin, overflow end} and
 // {Q0, Q1, Q3, det, 1/det}, the 2x2 system summed over the neighbours in order,
-// and per adjacency entry the neighbour and {ex, ey, L^3, 1/L^3} -- the same
-// expressions in the same order as the sequential sweep evaluates them.  Pads:
-// neighbour -1.  Overflow entries beyond n_ovf are reported through *bad.
+// and per adjacency entry the neighbour, {ex, ey} and (ecap further on) {L^3, 1/L^3} -- the same
+// expressions in the same order as the sequential sweep evaluates them.  Pads: neighbour N and
+// {1, 1, 2, 1}, which with a constant of 1 and a zero value gives the term 1 - (2 - 1) = +0 through
+// the same operations, its q0 = 1 in the fast division's range.  Overflow entries beyond n_ovf are reported through *bad.
 __global__ void __launch_bounds__(256) k_ct_geom(int N, const double* __restrict__ pts, const int32_t* __restrict__ nptr,
                                                  const int32_t* __restrict__ nidx, const int32_t* __restrict__ lidx,
                                                  const int32_t* __restrict__ slot_ovf, int n_ovf,
                                                  int4* __restrict__ slot_i, double* __restrict__ slot_v,
-                                                 int32_t* __restrict__ pe_q, double4* __restrict__ pe_geo,
-                                                 int32_t* __restrict__ bad) {
+                                                 int32_t* __restrict__ pe_q, double2* __restrict__ pe_geo,
+                                                 int64_t ecap, int32_t* __restrict__ bad) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= N) return;
     if (slot_ovf[N] > n_ovf) {
@@ -95,11 +101,14 @@ __global__ void __launch_bounds__(256) k_ct_geom(int N, const double* __restrict
         Q3 += 4 * ey * ey / L3;
         const int64_t e = ct_entry(N, t, k, slot_ovf);
         pe_q[e] = q;
-        pe_geo[e] = make_double4(ex, ey, L3, 1.0 / L3);
+        pe_geo[e] = make_double2(ex, ey);
+        pe_geo[ecap + e] = make_double2(L3, 1.0 / L3);
     }
     for (int k = deg; k < CT_SLOT; k++) {
-        pe_q[(int64_t)t * CT_SLOT + k] = -1;
-        pe_geo[(int64_t)t * CT_SLOT + k] = make_double4(0.0, 0.0, 1.0, 1.0);
+        const int64_t e = ct_entry(N, t, k, slot_ovf);
+        pe_q[e] = N;
+        pe_geo[e] = make_double2(1.0, 1.0);
+        pe_geo[ecap + e] = make_double2(2.0, 1.0);
     }
     const double Q2 = Q1;
     const double det = Q0 * Q3 - Q1 * Q2;
@@ -110,7 +119,7 @@ __global__ void __launch_bounds__(256) k_ct_geom(int N, const double* __restrict
     sv[2] = Q3;
     sv[3] = det;
     sv[4] = 1.0 / det;
-    sv[5] = 0.0;
+    sv[5] = __hiloint2double(slot_ovf[t + 1] - slot_ovf[t], p);   // for the pipelined sweeps: one record
 }
 
 // dens (N, Z) -> densT (Z, N): each slice contiguous
@@ -122,7 +131,7 @@ __global__ void __launch_bounds__(256) k_transpose_nz(const double* __restrict__
 }
 
 // The per-slice constant of every adjacency entry, 6 (f1 - f2) (the sweep's first
-// term, the same operation on the same values), A[z][entry]; 0 for pads.
+// term, the same operation on the same values), A[z][entry]; 1 for pads.
 __global__ void __launch_bounds__(256) k_ct_fdiff(const double* __restrict__ densT, int N, int Z, int64_t ecap,
                                                   const int4* __restrict__ slot_i, const int32_t* __restrict__ pe_q,
                                                   double* __restrict__ A) {
@@ -134,9 +143,9 @@ __global__ void __launch_bounds__(256) k_ct_fdiff(const double* __restrict__ den
     const double f1 = frow[si.x];
     double* Az = A + (int64_t)z * ecap;
     for (int k = 0; k < CT_SLOT; k++) {
-        const int64_t e = (int64_t)t * CT_SLOT + k;
+        const int64_t e = ct_entry(N, t, k, nullptr);
         const int q = pe_q[e];
-        Az[e] = (q >= 0) ? 6 * (f1 - frow[q]) : 0.0;
+        Az[e] = (q < N) ? 6 * (f1 - frow[q]) : 1.0;
     }
     for (int64_t e = (int64_t)N * CT_SLOT + si.y; e < (int64_t)N * CT_SLOT + si.z; e++)
         Az[e] = 6 * (f1 - frow[pe_q[e]]);
@@ -161,7 +170,8 @@ __device__ __forceinline__ bool ct_div_ok(double a, double q0) {
 // ((6 (f1 - f2) - 2 df2) ey) / L^3 with df2 = -ex y[q].x - ey y[q].y; exactly
 // rounded divisions (the IEEE division itself where the fast step's range test
 // fails).
-__device__ __forceinline__ double2 ct_terms(double a, const double4 g, const double2 yq) {
+__device__ __forceinline__ double2 ct_terms(double a, const double2 ge, const double2 gl, const double2 yq) {
+    const struct { double x, y, z, w; } g = {ge.x, ge.y, gl.x, gl.y};
     const double df2 = -g.x * yq.x - g.y * yq.y;
     const double u = a - 2 * df2;
     const double n0 = u * g.x, n1 = u * g.y;
@@ -205,7 +215,7 @@ constexpr int CT_SWEEP_UNROLL = 4;   // vertices per thread in flight in the end
 template <bool LDS_Y>
 __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients(
     int N, int Z, const int4* __restrict__ slot_i, const double* __restrict__ slot_v, const int32_t* __restrict__ pe_q,
-    const double4* __restrict__ pe_geo, const double* __restrict__ A, int64_t ecap, const int32_t* __restrict__ lptr,
+    const double2* __restrict__ pe_geo, const double* __restrict__ A, int64_t ecap, const int32_t* __restrict__ lptr,
     int n_levels, double tol, int maxiter, double* __restrict__ ybuf, double* __restrict__ grad_g,
     int32_t* __restrict__ iters_out) {
     extern __shared__ double4 s_dyn[];
@@ -239,20 +249,22 @@ __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients(
         return;
     }
     const uint32_t elast = (uint32_t)N * CT_SLOT - 1;
+    const uint32_t plane_k = (uint32_t)((k / CT_PIPE_LANES) * N * CT_PIPE_LANES + k % CT_PIPE_LANES);
     // this lane's adjacency entry and vertex, one level ahead; every load issued on
     // every lane (indices clamped into the arrays), so no load sits under a branch
     // and a use waits for its own loads only.  Byte offsets are 32-bit (the host
     // checks the arrays' sizes), so the loads take a scalar base and a 32-bit offset.
     int cq;
-    double4 cg;
+    double2 cg, cl;
     double ca;
     int4 vi;
     double vQ0, vQ1, vQ3, vdet, vrdet;
     auto load_level = [&](int l0, bool vert) {
         if (!vert) {
-            const uint32_t e = min((uint32_t)((l0 + j) * CT_SLOT + k), elast);
+            const uint32_t e = min(plane_k + (uint32_t)((l0 + j) * CT_PIPE_LANES), elast);
             cq = *(const int32_t*)((const char*)pe_q + (e << 2));
-            cg = *(const double4*)((const char*)pe_geo + (e << 5));
+            cg = *(const double2*)((const char*)pe_geo + (e << 4));
+            cl = *(const double2*)((const char*)(pe_geo + ecap) + (e << 4));
             ca = *(const double*)((const char*)Az + (e << 3));
         } else {
             const uint32_t t = min((uint32_t)(l0 + j), (uint32_t)(N - 1));
@@ -274,9 +286,9 @@ __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients(
         const bool act = j < lb1 - lb0;
         // the entry's terms
         if (act) {
-            const double2 yq = y[cq >= 0 ? cq : 0];
-            double2 tt = ct_terms(ca, cg, yq);
-            if (cq < 0) tt = make_double2(-0.0, -0.0);
+            const double2 yq = y[cq < N ? cq : 0];
+            double2 tt = ct_terms(ca, cg, cl, yq);
+            if (cq >= N) tt = make_double2(-0.0, -0.0);
             T[tid] = tt;
         }
         load_level(nb0, false);   // the next level's entries
@@ -294,7 +306,7 @@ __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients(
             }
             for (int64_t e = (int64_t)N * CT_SLOT + vi.y; e < (int64_t)N * CT_SLOT + vi.z; e++) {   // rare
                 const int q = pe_q[e];
-                const double2 tt = ct_terms(Az[e], pe_geo[e], y[q]);
+                const double2 tt = ct_terms(Az[e], pe_geo[e], pe_geo[ecap + e], y[q]);
                 s0 += tt.x;
                 s1 += tt.y;
             }
@@ -376,61 +388,94 @@ __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients(
 // reads, so the result is bit for bit the same.  A step runs the levels l = t - s P of the
 // sweeps in flight (at most ceil(levels / P)), one group of four lanes per vertex (two
 // entries each; otherwise as in k_ct_gradients).  Each update also writes its sweep's value to a ring of K sweeps in
-// global memory (y_hist) and raises the sweep's largest relative change (an LDS atomic max
-// on the non-negative doubles' bits); when a sweep's last level is done its change is
-// compared with tol, and on convergence (or at maxiter) the gradients are that sweep's ring
+// global memory (y_hist) and flags its sweep if its relative change is not below tol; a step
+// after a sweep's last level its flag is read, and on convergence (or at maxiter) the gradients are that sweep's ring
 // slot: the later sweeps in flight have overwritten some of the solution in LDS, but they
 // write other ring slots, and slot s is reused only by sweep s + K, which starts after the
-// check (K P > levels + P; the change slots likewise).
-// Step tables per residue r = t mod P (levels r, r + P, ...: their first slots, prefix
-// widths, and the map from a group to its level and place in it) are built in LDS at the start.  The workgroup holds four lanes for every vertex of
-// the widest step; the host checks that and the LDS before choosing this kernel.
+// check (K P > levels + P; the flags likewise).
+// Step tables per residue r = t mod P (levels r, r + P, ...: their prefix widths, and the map from
+// a group to its slot and its level's place among them) are built in LDS at the start.  The
+// workgroup holds four lanes for every vertex of the widest step; the host checks that and the LDS
+// before choosing this kernel.
+//
+// A step is one dependent chain -- barrier, neighbours' values from LDS, terms, in-order sums, 2 x 2
+// solve, the new value to LDS, barrier -- of a few waves, 1,008 times in a row at 91x81x101 (8 sweeps),
+// beside which a step's 36 KB of inputs come from L2.  So: inputs in planes that the lanes read in whole
+// lines, two steps ahead into two register sets, slots located three steps ahead; terms exchanged by
+// DPP (no LDS round trip); pads that need no masks; one range test for a lane's divisions, each one's
+// own only if that fails; and a convergence test that only asks whether some change is not below tol,
+// which each vertex decides a step later, while the next step's values are on their way, without a
+// division unless it is close.  1.37 -> 1.02 ms at 91x81x101.  Measured and not kept: two lanes per
+// vertex (1.11), the loads at the start or at the end of a step (1.19, 1.17), one test and one rare branch
+// for the terms and the solve together (1.07), streaming loads of the constants (1.30).  Without any
+// loads a step still takes three quarters of its time.
 constexpr int CT_MAX_K = 16;
-constexpr int CT_PIPE_LANES = 4;   // lanes per vertex in the pipelined sweeps (two entries each)
 
-__global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients_pipe(
+// the value of lane I of this lane's group, for the group's first lane
+template <int I>
+__device__ __forceinline__ double ct_lane(double v) {
+    if (I == 0) return v;
+    constexpr int ctrl = I * 0x55;   // quad_perm: lane I of every four
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+template <int E>
+__device__ __forceinline__ void ct_sum(const double2 (&t)[CT_PIPE_ENT], double& s0, double& s1) {
+    if constexpr (E < CT_SLOT) {
+        s0 += ct_lane<E % CT_PIPE_LANES>(t[E / CT_PIPE_LANES].x);
+        s1 += ct_lane<E % CT_PIPE_LANES>(t[E / CT_PIPE_LANES].y);
+        ct_sum<E + 1>(t, s0, s1);
+    }
+}
+
+// inputs of one vertex update: the lane's adjacency entries, the vertex's record
+struct CtIn {
+    int q[CT_PIPE_ENT];
+    double2 g[CT_PIPE_ENT], l[CT_PIPE_ENT];   // {ex, ey}, {L^3, 1 / L^3}
+    double a[CT_PIPE_ENT];
+    double Q0, Q1, Q3, det, rdet;
+    int p, ovf, slot, ring;
+    bool act;
+};
+
+// NT: threads the registers are sized for; both input sets fit without spills at 512 (steps of up to
+// 128 vertices), wider steps take 1024
+template <int NT>
+__global__ void __launch_bounds__(NT) k_ct_gradients_pipe(
     int N, int Z, const int4* __restrict__ slot_i, const double* __restrict__ slot_v, const int32_t* __restrict__ pe_q,
-    const double4* __restrict__ pe_geo, const double* __restrict__ A, int64_t ecap, const int32_t* __restrict__ lptr,
+    const double2* __restrict__ pe_geo, const double* __restrict__ A, int64_t ecap, const int32_t* __restrict__ lptr,
     int n_levels, int P, int K, int W, double tol, int maxiter, double* __restrict__ y_hist,
     double* __restrict__ grad_g, int32_t* __restrict__ iters_out) {
     extern __shared__ double4 s_dyn[];
-    __shared__ unsigned long long s_err[CT_MAX_K];
+    __shared__ int s_open[CT_MAX_K];   // the sweep of this ring slot has a change that is not below tol
     __shared__ int s_bad;
     const int z = blockIdx.x;
     const int nthr = blockDim.x;
     const int tid = threadIdx.x;
-    const int j = tid / CT_PIPE_LANES, k = tid % CT_PIPE_LANES;   // lane k holds entries k and k + 4
+    const int j = tid / CT_PIPE_LANES, k = tid % CT_PIPE_LANES;
     const double* Az = A + (int64_t)z * ecap;
     double2* hz = (double2*)(y_hist + (int64_t)z * K * N * 2);
     const int KM = (n_levels + P - 1) / P;   // levels per residue, at most
-    // LDS: [solution N double2] [terms 8 per group double2] [level slot pointers n+1] [per residue:
-    // level count P, first slots P KM, prefix widths P (KM + 1), step map P W (16-bit)]
+    // LDS: [solution N double2, a zero for the pads] [per residue: prefix widths P (KM + 1)] [step map P W: slot (16-bit)]
+    // [the slot's level: its place among the residue's (8-bit)]
     double2* y = (double2*)s_dyn;
-    double2* T = y + N;   // the terms of group g's entries at T[g CT_SLOT .. g CT_SLOT + 7]
-    int32_t* s_lptr = (int32_t*)(T + (nthr / CT_PIPE_LANES) * CT_SLOT);
-    int32_t* s_cnt = s_lptr + n_levels + 1;
-    int32_t* s_start = s_cnt + P;
-    int32_t* s_pre = s_start + P * KM;
-    uint16_t* s_map = (uint16_t*)(s_pre + P * (KM + 1));   // (level k of the residue) << 12 | index in the level
-    for (int i = tid; i < N; i += nthr) y[i] = make_double2(0.0, 0.0);
+    int32_t* s_pre = (int32_t*)(y + N + 1);
+    uint16_t* s_map = (uint16_t*)(s_pre + P * (KM + 1));
+    uint8_t* s_kk = (uint8_t*)(s_map + P * W);
+    int32_t* s_lptr = (int32_t*)s_dyn;   // while the tables are built (n_levels <= N)
     for (int i = tid; i <= n_levels; i += nthr) s_lptr[i] = lptr[i];
-    if (tid < CT_MAX_K) s_err[tid] = 0ull;
+    if (tid < CT_MAX_K) s_open[tid] = 0;
     if (tid == 0) s_bad = 0;
     __syncthreads();
     for (int r = tid; r < P; r += nthr) {
-        int c = 0, acc = 0;
-        for (int l = r; l < n_levels; l += P, c++) {
-            s_start[r * KM + c] = s_lptr[l];
-            s_pre[r * (KM + 1) + c] = acc;
-            acc += s_lptr[l + 1] - s_lptr[l];
+        int acc = 0;
+        for (int kk = 0, l = r; kk < KM; kk++, l += P) {
+            s_pre[r * (KM + 1) + kk] = acc;
+            if (l < n_levels) acc += s_lptr[l + 1] - s_lptr[l];
         }
-        s_pre[r * (KM + 1) + c] = acc;
-        s_cnt[r] = c;
+        s_pre[r * (KM + 1) + KM] = acc;
         if (acc * CT_PIPE_LANES > nthr || acc > W) s_bad = 1;   // a step wider than the workgroup: refuse
-        else
-            for (int l = r, kk = 0; l < n_levels; l += P, kk++)
-                for (int i = 0; i < s_lptr[l + 1] - s_lptr[l]; i++)
-                    s_map[r * W + s_pre[r * (KM + 1) + kk] + i] = (uint16_t)((kk << 12) | i);
     }
     __syncthreads();
     if (s_bad) {
@@ -440,148 +485,186 @@ __global__ void __launch_bounds__(CT_MAX_THREADS) k_ct_gradients_pipe(
         }
         return;
     }
-    // the vertex of this lane's group at step t = q P + r (false: none) and its sweep; the
-    // prefix widths of the residue are read together and counted, no dependent search
-    auto locate = [&](int q, int r, int& slot, int& sweep) -> bool {
-        if (q >= KM - 1 && q < maxiter) {   // every level of every residue in flight: the map directly
-            if (j >= s_pre[r * (KM + 1) + s_cnt[r]]) return false;
-            const int e = s_map[r * W + j];
-            slot = s_start[r * KM + (e >> 12)] + (e & 4095);
-            sweep = q - (e >> 12);
-            return true;
-        }
-        const int cnt = s_cnt[r];
-        const int khi = min(cnt - 1, q);                 // levels r + k P <= t
-        const int klo = max(0, q - maxiter + 1);         // sweeps (t - l) / P < maxiter
-        if (klo > khi) return false;
-        const int32_t* pre = s_pre + r * (KM + 1);
-        const int g = j + pre[klo];
-        if (g >= pre[khi + 1]) return false;
-        const int e = s_map[r * W + g];
-        slot = s_start[r * KM + (e >> 12)] + (e & 4095);
-        sweep = q - (e >> 12);
-        return true;
-    };
-    const uint32_t elast = (uint32_t)N * CT_SLOT - 1;
-    int cq, cq2;
-    double4 cg, cg2;
-    double ca, ca2;
-    int4 vi;
-    double vQ0, vQ1, vQ3, vdet, vrdet;
-    auto load_entry = [&](int slot) {
-        const uint32_t e = min((uint32_t)(slot * CT_SLOT + k), elast);
-        const uint32_t e2 = min(e + CT_PIPE_LANES, elast);
-        cq = *(const int32_t*)((const char*)pe_q + (e << 2));
-        cq2 = *(const int32_t*)((const char*)pe_q + (e2 << 2));
-        cg = *(const double4*)((const char*)pe_geo + (e << 5));
-        cg2 = *(const double4*)((const char*)pe_geo + (e2 << 5));
-        ca = *(const double*)((const char*)Az + (e << 3));
-        ca2 = *(const double*)((const char*)Az + (e2 << 3));
-    };
-    auto load_vert = [&](int slot) {
-        const uint32_t t = min((uint32_t)slot, (uint32_t)(N - 1));
-        vi = *(const int4*)((const char*)slot_i + (t << 4));
-        const double* sv = (const double*)((const char*)slot_v + t * 48u);
-        vQ0 = sv[0];
-        vQ1 = sv[1];
-        vQ3 = sv[2];
-        vdet = sv[3];
-        vrdet = sv[4];
-    };
-    // steps t (current) and t + 1 located; t + 2 is located during step t, after its updates
-    int slot = 0, sweep = 0, slot1 = 0, sweep1 = 0;
-    int q2 = 2 / P, r2 = 2 % P;   // t + 2 = q2 P + r2
-    bool act = locate(0, 0, slot, sweep);
-    bool act1 = locate(1 / P, 1 % P, slot1, sweep1);
-    load_entry(act ? slot : 0);
-    load_vert(act ? slot : 0);
-    int iters = 0, fin = 0;
-    for (int t = 0;; t++) {
-        // the entry's terms
-        if (act) {
-            const double2 yq = y[cq >= 0 ? cq : 0], yq2 = y[cq2 >= 0 ? cq2 : 0];
-            double2 tt = ct_terms(ca, cg, yq), tt2 = ct_terms(ca2, cg2, yq2);
-            if (cq < 0) tt = make_double2(-0.0, -0.0);
-            if (cq2 < 0) tt2 = make_double2(-0.0, -0.0);
-            T[j * CT_SLOT + k] = tt;
-            T[j * CT_SLOT + k + CT_PIPE_LANES] = tt2;
-        }
-        load_entry(act1 ? slot1 : 0);   // the next step's entry
-        asm volatile("" ::: "memory");
-        // the group's first lane: in-order sums, overflow entries, solve, change, ring
-        if (act && k == 0) {
-            double2 tk[CT_SLOT];
-#pragma unroll
-            for (int i = 0; i < CT_SLOT; i++) tk[i] = T[j * CT_SLOT + i];
-            const double2 yo = y[vi.x];
-            double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-            for (int i = 0; i < CT_SLOT; i++) {
-                s0 += tk[i].x;
-                s1 += tk[i].y;
-            }
-            for (int64_t e = (int64_t)N * CT_SLOT + vi.y; e < (int64_t)N * CT_SLOT + vi.z; e++) {   // rare
-                const int q = pe_q[e];
-                const double2 tt = ct_terms(Az[e], pe_geo[e], y[q]);
-                s0 += tt.x;
-                s1 += tt.y;
-            }
-            const double Q2 = vQ1;
-            const double n0 = vQ3 * s0 - vQ1 * s1;
-            const double n1 = -Q2 * s0 + vQ0 * s1;
-            const double q0 = n0 * vrdet, q1 = n1 * vrdet;
-            double r0 = ct_div_fast(n0, vdet, vrdet, q0);
-            double r1 = ct_div_fast(n1, vdet, vrdet, q1);
-            if (!((vdet > 0.0) & ct_div_ok(n0, q0) & ct_div_ok(n1, q1))) {   // rare: exactly rounded either way
-                r0 = n0 / vdet;
-                r1 = n1 / vdet;
-            }
-            const double2 yn = make_double2(-r0, -r1);
-            y[vi.x] = yn;
-            hz[(int64_t)(sweep % K) * N + vi.x] = yn;
-            // scipy's change: max(|y_old + r|) / max(1, max|r|)
-            const double a0 = fabs(yo.x + r0), a1 = fabs(yo.y + r1);
-            const double m0 = fabs(r0), m1 = fabs(r1);
-            const double num = (a0 > a1) ? a0 : a1;
-            const double mr = (m0 > m1) ? m0 : m1;
-            const double den = (1.0 > mr) ? 1.0 : mr;
-            const double ch = num / den;
-            atomicMax(s_err + sweep % K, (unsigned long long)__double_as_longlong(ch));
-        }
-        load_vert(act1 ? slot1 : 0);   // the next step's vertex
-        int slot2 = 0, sweep2 = 0;
-        const bool act2 = locate(q2, r2, slot2, sweep2);
-        if (++r2 == P) {
-            r2 = 0;
-            q2++;
-        }
-        ct_barrier_lds();
-        act = act1;
-        slot = slot1;
-        sweep = sweep1;
-        act1 = act2;
-        slot1 = slot2;
-        sweep1 = sweep2;
-        // a sweep whose last level was this step: its convergence test
-        const int tl = t - (n_levels - 1);
-        if (tl >= 0 && tl % P == 0) {
-            const int sc = tl / P;
-            const double m = __longlong_as_double((long long)s_err[sc % K]);
-            if (m < tol) {
-                iters = sc + 1;
-                fin = sc;
-                break;
-            }
-            if (sc + 1 >= maxiter) {
-                fin = sc;
-                break;
-            }
-            __syncthreads();   // every thread has read the slot before it is cleared
-            if (tid == 0) s_err[sc % K] = 0ull;
+    for (int l = tid; l < n_levels; l += nthr) {
+        const int r = l % P, kk = l / P, s0 = s_lptr[l], at = r * W + s_pre[r * (KM + 1) + kk];
+        for (int i = 0; i < s_lptr[l + 1] - s0; i++) {
+            s_map[at + i] = (uint16_t)(s0 + i);
+            s_kk[at + i] = (uint8_t)kk;
         }
     }
+    __syncthreads();
+    for (int i = tid; i <= N; i += nthr) y[i] = make_double2(0.0, 0.0);
+    __syncthreads();
+    // the slot of this lane's group at step t = q P + r (act: there is one) and its sweep's ring
+    // slot; qK = q mod K
+    struct Loc {
+        int slot, ring;
+        bool act;
+    };
+    auto locate = [&](int q, int r, int qK) -> Loc {
+        const int32_t* pre = s_pre + r * (KM + 1);
+        const int khi = min(KM - 1, q);                       // levels r + k P <= t
+        const int klo = max(0, q - maxiter + 1);              // sweeps (t - l) / P < maxiter
+        int g = j;
+        if (klo > 0) g += pre[min(klo, KM)];
+        const int i = r * W + min(g, W - 1);
+        const int slot = s_map[i], kk = s_kk[i];
+        Loc L;
+        L.act = (klo <= khi) & (g < pre[khi + 1]);
+        L.slot = L.act ? slot : 0;
+        L.ring = qK - kk + ((qK < kk) ? K : 0);
+        return L;
+    };
+    // (32-bit byte offsets: N is below 2^14 when the solution fits the LDS)
+    auto load_entries = [&](CtIn& b, int slot) {
+        const uint32_t e = (uint32_t)(slot * CT_PIPE_LANES + k), plane = (uint32_t)(N * CT_PIPE_LANES);
+        const char *cq = (const char*)pe_q + (e << 2), *cg = (const char*)pe_geo + (e << 4),
+                   *cl = (const char*)(pe_geo + ecap) + (e << 4), *ca = (const char*)Az + (e << 3);
+#pragma unroll
+        for (int i = 0; i < CT_PIPE_ENT; i++) {
+            b.q[i] = *(const int32_t*)(cq + i * plane * 4);
+            b.g[i] = *(const double2*)(cg + i * plane * 16);
+            b.l[i] = *(const double2*)(cl + i * plane * 16);
+            b.a[i] = *(const double*)(ca + i * plane * 8);
+        }
+    };
+    auto load_vert = [&](CtIn& b, const Loc& L) {
+        const double2* sv = (const double2*)((const char*)slot_v + __umul24((uint32_t)L.slot, 48u));
+        const double2 v0 = sv[0], v1 = sv[1], v2 = sv[2];
+        b.Q0 = v0.x;
+        b.Q1 = v0.y;
+        b.Q3 = v1.x;
+        b.det = v1.y;
+        b.rdet = v2.x;
+        b.p = __double2loint(v2.y);
+        b.ovf = __double2hiint(v2.y);
+        b.slot = L.slot;
+        b.ring = L.ring;
+        b.act = L.act;
+    };
+    // surely below / surely not below tol without the division (1e-9 against its half ulp)
+    const double tol_lo = tol * (1.0 - 1e-9), tol_hi = tol * (1.0 + 1e-9);
+    bool ch_on = false;   // the last step's update of this lane: old value, r, ring slot
+    double2 ch_yo = make_double2(0.0, 0.0);
+    double ch_r0 = 0.0, ch_r1 = 0.0;
+    int ch_ring = 0;
+    int q3 = 3 / P, r3 = 3 % P, qK3 = q3 % K;   // t + 3 = q3 P + r3
+    CtIn in0, in1;
+    Loc ahead;   // step t + 2
+    {
+        const Loc L0 = locate(0, 0, 0), L1 = locate(1 / P, 1 % P, (1 / P) % K);
+        ahead = locate(2 / P, 2 % P, (2 / P) % K);
+        load_entries(in0, L0.slot);
+        load_vert(in0, L0);
+        load_entries(in1, L1.slot);
+        load_vert(in1, L1);
+        // the first steps' inputs are in place, so that inside the loop a step waits for its own only
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    }
+    int iters = 0, fin = 0;
+    int check = n_levels, sc = 0, scK = 0;   // step at whose end sweep sc is tested; sc mod K
+    // one step on the inputs b, which then take those of step t + 2; true when the sweeps have ended
+    auto step = [&](CtIn& b, int t) -> bool {
+        double2 yq[CT_PIPE_ENT];
+#pragma unroll
+        for (int i = 0; i < CT_PIPE_ENT; i++) yq[i] = y[b.q[i]];
+        const double2 yo = y[b.p];
+        const Loc next = locate(q3, r3, qK3);
+        if (++r3 == P) {
+            r3 = 0;
+            q3++;
+            if (++qK3 == K) qK3 = 0;
+        }
+        // scipy's change of the last step's vertex: max(|y_old + r|) / max(1, max|r|) against tol
+        if (ch_on) {
+            const double c0 = fabs(ch_yo.x + ch_r0), c1 = fabs(ch_yo.y + ch_r1);
+            const double m0 = fabs(ch_r0), m1 = fabs(ch_r1);
+            const double num = (c0 > c1) ? c0 : c1;
+            const double mr = (m0 > m1) ? m0 : m1;
+            const double den = (1.0 > mr) ? 1.0 : mr;
+            if (!(num < tol_lo * den)) {
+                bool open = true;
+                if (__builtin_expect(!(num > tol_hi * den), 0)) open = !(num / den < tol);   // close to tol, or not a number
+                if (open) s_open[ch_ring] = 1;
+            }
+        }
+        // the terms: ct_terms with one range test for the lane's entries, which an exact zero or a value
+        // out of range fails (a NaN gives NaN by either division)
+        double2 t4[CT_PIPE_ENT];
+        double lo = HUGE_VAL, hi = 0.0;
+#pragma unroll
+        for (int i = 0; i < CT_PIPE_ENT; i++) {
+            const double df2 = -b.g[i].x * yq[i].x - b.g[i].y * yq[i].y;
+            const double u = b.a[i] - 2 * df2;
+            const double n0 = u * b.g[i].x, n1 = u * b.g[i].y;
+            const double q0 = n0 * b.l[i].y, q1 = n1 * b.l[i].y;
+            t4[i].x = ct_div_fast(n0, b.l[i].x, b.l[i].y, q0);
+            t4[i].y = ct_div_fast(n1, b.l[i].x, b.l[i].y, q1);
+            lo = fmin(lo, fmin(fabs(q0), fabs(q1)));
+            hi = fmax(hi, fmax(fabs(q0), fabs(q1)));
+        }
+        if (!((lo >= 0x1p-900) & (hi <= 0x1p+900))) {
+#pragma unroll
+            for (int i = 0; i < CT_PIPE_ENT; i++) t4[i] = ct_terms(b.a[i], b.g[i], b.l[i], yq[i]);
+        }
+        load_entries(b, ahead.slot);
+        double s0 = 0.0, s1 = 0.0;
+        ct_sum<0>(t4, s0, s1);   // in order
+        ch_on = b.act && k == 0;
+        if (ch_on) {
+            if (__builtin_expect(b.ovf > 0, 0)) {
+                const int4 vi = slot_i[b.slot];
+                for (int64_t e = (int64_t)N * CT_SLOT + vi.y; e < (int64_t)N * CT_SLOT + vi.z; e++) {
+                    const int q = pe_q[e];
+                    const double2 tt = ct_terms(Az[e], pe_geo[e], pe_geo[ecap + e], y[q]);
+                    s0 += tt.x;
+                    s1 += tt.y;
+                }
+            }
+            const double n0 = b.Q3 * s0 - b.Q1 * s1;
+            const double n1 = -b.Q1 * s0 + b.Q0 * s1;
+            const double d0 = n0 * b.rdet, d1 = n1 * b.rdet;
+            double r0 = ct_div_fast(n0, b.det, b.rdet, d0);
+            double r1 = ct_div_fast(n1, b.det, b.rdet, d1);
+            if (!((b.det > 0.0) & (fmin(fabs(d0), fabs(d1)) >= 0x1p-900) & (fmax(fabs(d0), fabs(d1)) <= 0x1p+900))) {
+                if (!((b.det > 0.0) & ct_div_ok(n0, d0) & ct_div_ok(n1, d1))) {   // rare: exactly rounded either way
+                    r0 = n0 / b.det;
+                    r1 = n1 / b.det;
+                }
+            }
+            const double2 yn = make_double2(-r0, -r1);
+            y[b.p] = yn;
+            *(double2*)((char*)hz + ((__umul24((uint32_t)b.ring, (uint32_t)N) + (uint32_t)b.p) << 4)) = yn;
+            ch_yo = yo;
+            ch_r0 = r0;
+            ch_r1 = r1;
+            ch_ring = b.ring;
+        }
+        load_vert(b, ahead);
+        ahead = next;
+        ct_barrier_lds();
+        // a sweep whose last level was the step before: its convergence test (its flags are in place)
+        if (t == check) {
+            const bool open = s_open[scK] != 0;
+            if (!open || sc + 1 >= maxiter) {
+                iters = open ? 0 : sc + 1;
+                fin = scK;
+                return true;
+            }
+            __syncthreads();   // every thread has read the slot before it is cleared
+            if (tid == 0) s_open[scK] = 0;
+            check += P;
+            sc++;
+            if (++scK == K) scK = 0;
+        }
+        return false;
+    };
+    for (int t = 0;; t += 2) {
+        if (step(in0, t)) break;
+        if (step(in1, t + 1)) break;
+    }
     __syncthreads();   // the ring writes of every thread are complete
-    const double2* src = hz + (int64_t)(fin % K) * N;
+    const double2* src = hz + (int64_t)fin * N;
     double2* dst = (double2*)(grad_g + (int64_t)z * N * 2);
     for (int i = tid; i < N; i += nthr) dst[i] = src[i];
     if (tid == 0) iters_out[z] = iters;
@@ -986,7 +1069,7 @@ extern "C" int hd_scatter(double* dens, int M, int Q, int Z, int G, const double
     int4* slot_i = (int4*)p;          p += align256((size_t)N * 16);
     double* slot_v = (double*)p;      p += align256((size_t)N * 6 * 8);
     int32_t* pe_q = (int32_t*)p;      p += align256((size_t)ecap * 4);
-    double4* pe_geo = (double4*)p;    p += align256((size_t)ecap * 32);
+    double2* pe_geo = (double2*)p;    p += align256((size_t)ecap * 32);
     double* ybuf = (double*)p;        p += align256((size_t)N * Z * 2 * 8);
     double* fdiff = (double*)p;       p += align256((size_t)Z * ecap * 8);
     double* y_hist = (double*)p;
@@ -995,7 +1078,7 @@ extern "C" int hd_scatter(double* dens, int M, int Q, int Z, int G, const double
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, bad, 1);
     hipLaunchKernelGGL(k_ct_slots, dim3(1), dim3(1024), 0, st, N, nbr_ptr, levels_idx, slot_ovf);
     hipLaunchKernelGGL(k_ct_geom, dim3((unsigned)cdiv(N, 256)), dim3(256), 0, st, N, pts, nbr_ptr, nbr_idx, levels_idx,
-                       slot_ovf, n_ovf, slot_i, slot_v, pe_q, pe_geo, bad);
+                       slot_ovf, n_ovf, slot_i, slot_v, pe_q, pe_geo, ecap, bad);
     hipLaunchKernelGGL(k_transpose_nz, dim3((unsigned)cdiv((int64_t)N * Z, 256)), dim3(256), 0, st, dens, N, Z, densT);
     hipLaunchKernelGGL(k_ct_fdiff, dim3((unsigned)cdiv((int64_t)N * Z, 256)), dim3(256), 0, st, densT, N, Z, ecap,
                        slot_i, pe_q, fdiff);
@@ -1013,17 +1096,16 @@ extern "C" int hd_scatter(double* dens, int M, int Q, int Z, int G, const double
     if (K > 0 && max_step_width > 0) {
         const int nthr_p = (int)(((int64_t)max_step_width * CT_PIPE_LANES + 63) / 64 * 64);
         const int KM = (n_levels + sweep_period - 1) / sweep_period;
-        const size_t lds_p = (size_t)N * 16 + (size_t)(nthr_p / CT_PIPE_LANES) * CT_SLOT * 16 +
-                             (size_t)(n_levels + 1) * 4 + (size_t)sweep_period * (1 + KM + KM + 1) * 4 +
-                             (size_t)sweep_period * max_step_width * 2 + 256;
-        if (nthr_p <= CT_MAX_THREADS && max_level_width < 4096 && lds_p <= (size_t)max_lds) {
+        const size_t lds_p = (size_t)(N + 1) * 16 + (size_t)sweep_period * (KM + 1) * 4 +
+                             (size_t)sweep_period * max_step_width * 3 + 256;
+        if (nthr_p <= CT_MAX_THREADS && N < 16384 && n_levels <= N && lds_p <= (size_t)max_lds) {
+            const auto kfn_p = (nthr_p <= 512) ? k_ct_gradients_pipe<512> : k_ct_gradients_pipe<CT_MAX_THREADS>;
             if (lds_p > 65536) {
-                he = hipFuncSetAttribute((const void*)k_ct_gradients_pipe, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)lds_p);
+                he = hipFuncSetAttribute((const void*)kfn_p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_p);
                 if (he != hipSuccess)
                     return set_error(HD_ERR_HIP, "hd_scatter: LDS attribute: %s", hipGetErrorString(he));
             }
-            hipLaunchKernelGGL(k_ct_gradients_pipe, dim3(Z), dim3(nthr_p), lds_p, st, N, Z, slot_i, slot_v, pe_q,
+            hipLaunchKernelGGL(kfn_p, dim3(Z), dim3(nthr_p), lds_p, st, N, Z, slot_i, slot_v, pe_q,
                                pe_geo, fdiff, ecap, levels_ptr, n_levels, sweep_period, K, max_step_width, tol, maxiter,
                                y_hist, grad, iters_out);
             int rcp = check_launch("k_ct_gradients_pipe");
