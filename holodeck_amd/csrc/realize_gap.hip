@@ -697,7 +697,7 @@ __device__ __forceinline__ void gz_entries(gz_lds_u32* hi, gz_lds_u32* lo, int m
 }
 
 template <int G>
-__device__ __noinline__ void gz_build(gz_lrec rec, gz_lds_u32* hi, bool on, int gl) {
+__device__ __forceinline__ void gz_build(gz_lrec rec, gz_lds_u32* hi, bool on, int gl) {
     const int n = on ? rec->n : 0, kb = rec->kb, kt = on ? rec->kt : kb;
     gz_lds_u32* lo = hi + n;
     const int nb = kt + n - kb;          // counts summed
@@ -729,7 +729,7 @@ struct GzPart {
     int j0, m;                 // this lane's counts
 };
 
-__device__ __noinline__ GzPart gz_part_sum(gz_lrec rec, gz_lds_u32* hi, int j_lo, int j_hi, int lane,
+__device__ __forceinline__ GzPart gz_part_sum(gz_lrec rec, gz_lds_u32* hi, int j_lo, int j_hi, int lane,
                                            double* s_part) {
     const int s = ((j_hi - j_lo + 63) >> 6) | 1;   // odd, as in gz_build
     GzPart P;
@@ -748,7 +748,7 @@ __device__ __noinline__ GzPart gz_part_sum(gz_lrec rec, gz_lds_u32* hi, int j_lo
 }
 
 // part: its index; s_part: the sums of the table's part 0 (2 doubles each)
-__device__ __noinline__ void gz_part_write(gz_lrec rec, gz_lds_u32* hi, GzPart P, int part,
+__device__ __forceinline__ void gz_part_write(gz_lrec rec, gz_lds_u32* hi, GzPart P, int part,
                                            const double* s_part) {
     double scale = rec->p0, base = 0.0;
     for (int q = 0; q < part; q++) {
@@ -998,6 +998,49 @@ __device__ __forceinline__ void gz_draw2(const GzTab& ta, const GzTab& tb, Words
     cb = (tb.n > 0) ? gz_count(tb, jb, xb, wb, hwb, rs) : 0;
 }
 
+// Four draws from tables that all have entries, their searches interleaved: the words and counts of two
+// gz_draw2 in a row where every candidate of the wave stands, else false and the words are not taken.
+// (A step of a finished search, len = 1, leaves it as it is, so the four run as long as the longest.)
+// A search is a chain of LDS round trips; in pairs they took a third to three fifths of the launch,
+// most where few realizations leave few waves.  With the table builds inline, whose calls had spilled
+// what lives across them (a fifth of this gain): 91x81x101 x 40, R = 500 6.69 -> 6.09 ms, 61x51x41 x 20,
+// R = 100 with parameters 2.30 -> 2.14, library samples 0.95 + 0.89 -> 0.86 + 0.79, eccentric
+// realizations 24.0 -> 22.8.  Six at a time measured the same within 3 %, eight slower (7.5 ms in the
+// first of these: the records' scalars spill).
+template <class Words>
+__device__ __forceinline__ bool gz_draw4(const GzTab (&t)[4], Words& rs, int (&k)[4]) {
+    const Words before = rs;
+    GzSearch s[4];
+    int len = 1;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        gz_search_start(s[i], t[i].hi, t[i].n, rs.next());
+        len = max(len, t[i].n);
+    }
+    while (len > 1) {
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = s[i].p[s[i].len >> 1];   // in flight together
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int half = s[i].len >> 1;
+            s[i].p = (v[i] < s[i].x) ? s[i].p + half : s[i].p;
+            s[i].len -= half;
+        }
+        len -= len >> 1;
+    }
+    bool fine = true;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        bool stands;
+        k[i] = gz_candidate(t[i], s[i].p, s[i].x, stands);
+        fine &= stands;
+    }
+    if (__builtin_amdgcn_ballot_w64(!fine) == 0ull) return true;
+    rs = before;
+    return false;
+}
+
 // The table of a staged header (the header is the same for the whole wave: its
 // fields go to scalar registers); present = false gives an empty table.
 __device__ __forceinline__ GzTab gz_tab(const uint32_t* tab, const BRec* b, bool present) {
@@ -1211,7 +1254,30 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
                     const int cd = min(c1, nd);
                     const DRec* rec = A.drec + rreg;
                     {
+                        int pairs_to = c;   // records before this are drawn in pairs
                         for (int i = c; i < cd; i += 2) {
+                            if (i >= pairs_to && i + 4 <= cd) {
+                                GzDraw d[4];
+                                GzTab t[4];
+                                int k[4], shortest = 1;
+#pragma unroll
+                                for (int q = 0; q < 4; q++) {
+                                    d[q] = gz_load_draw(rec + i + q);
+                                    t[q] = gz_tab_rec(tab, d[q], base, brec + (i + q - c), true);
+                                    shortest = min(shortest, d[q].n);
+                                }
+                                if (shortest > 0 && gz_draw4(t, rs, k)) {
+                                    const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
+#pragma unroll
+                                    for (int q = 0; q < 4; q++) {
+                                        acc.add((double)k[q], d[q].h, d[q].word, par + q, pstride, A.npar, L);
+                                        if (REC) gz_record(A, d[q].word, f, r, (double)k[q], false);
+                                    }
+                                    i += 2;
+                                    continue;
+                                }
+                                pairs_to = i + 4;
+                            }
                             const bool hb = i + 1 < cd;
                             const GzDraw ra = gz_load_draw(rec + i), rb = gz_load_draw(rec + (hb ? i + 1 : i));
                             const GzTab ta = gz_tab_rec(tab, ra, base, brec + (i - c), true);
