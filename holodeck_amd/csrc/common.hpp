@@ -148,6 +148,45 @@ __device__ __forceinline__ double cosmo_dcom(const Cosmo& C, double z) {
     return v * C.d_hubble;
 }
 
+// A 256-thread block's item of a kernel over (mass bin, ratio bin, redshift bins, frequency): one (mass,
+// ratio) bin mq per run of blocks, BIN_ZC redshift bins from z0 at frequency ff per thread, frequency
+// fastest; and the values of an (M, Q, Z, F) array at their corners, v[2 i + j][k] at mass mm + i, ratio
+// qq + j, redshift z0 + k (past the grid's end: the last one), loaded together.
+constexpr int BIN_ZC = 4;
+struct BinItem {
+    int mq, mm, qq, z0, ff;
+    bool live;
+};
+__device__ __forceinline__ BinItem bin_item(int Q, int Z, int F) {
+    const uint32_t per_mq = (uint32_t)((Z - 1 + BIN_ZC - 1) / BIN_ZC) * (uint32_t)F;
+    const uint32_t nchunk = (per_mq + 255u) / 256u;
+    BinItem it;
+    it.mq = (int)(blockIdx.x / nchunk);   // uniform
+    it.mm = it.mq / (Q - 1);
+    it.qq = it.mq - it.mm * (Q - 1);
+    const uint32_t loc = (blockIdx.x - (uint32_t)it.mq * nchunk) * 256u + threadIdx.x;
+    it.live = loc < per_mq;
+    const uint32_t zc = loc / (uint32_t)F;
+    it.z0 = (int)zc * BIN_ZC;
+    it.ff = (int)(loc - zc * (uint32_t)F);
+    return it;
+}
+__device__ __forceinline__ void bin_corners(const double* __restrict__ a, const BinItem& it, int Q, int Z, int F,
+                                            double (&v)[4][BIN_ZC + 1]) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const double* p = a + (((int64_t)(it.mm + (c >> 1)) * Q + (it.qq + (c & 1))) * Z + it.z0) * F + it.ff;
+#pragma unroll
+        for (int k = 0; k <= BIN_ZC; k++) v[c][k] = p[(int64_t)min(k, Z - 1 - it.z0) * F];
+    }
+}
+
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// blocks of such a kernel; -1: more outputs than 32-bit numbers take, or than a launch of one each
+inline int64_t bin_blocks(int M, int Q, int Z, int F) {
+    const int64_t per_mq = (int64_t)(Z - 1) * F, mq = (int64_t)(M - 1) * (Q - 1);
+    if (per_mq > 0xffffffffll || mq * cdiv(per_mq, 256) > 0x7fffffffll) return -1;
+    return mq * cdiv(cdiv(Z - 1, BIN_ZC) * F, 256);
+}
 
 }  // namespace hd

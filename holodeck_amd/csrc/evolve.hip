@@ -603,36 +603,37 @@ __global__ void __launch_bounds__(DBN_THREADS, 5) k_dbn_2pwl(EvoConsts K, const 
 
 // ---------------------------------------------------------------------------
 // 3D trapezoid x 1D Riemann integration (sam_cyutils.pyx:166-216).
-// One thread per output (m,q,z,f); corner order and operation order follow
-// the reference loop.
+// Corner order and operation order follow the reference loop.
 // ---------------------------------------------------------------------------
-// block b: (mass, ratio) bin b / nchunk, chunk b % nchunk of its 256-output chunks of (redshift
-// bin, frequency) -- the chunks of a bin consecutive, as the corner rows they share; a thread
-// decodes its output with one 32-bit division (the flat decode took three 64-bit ones)
+// block b: (mass, ratio) bin b / nchunk, chunk b % nchunk of its (redshift group, frequency) items -- the
+// chunks of a bin consecutive, as the corner rows they share.  A thread takes BIN_ZC redshift bins in
+// a row, whose corners it loads together: five loads per output instead of eight, one decoding and one
+// set of addresses (0.21 -> 0.18 ms at 91x81x101 x 40; 0.47 GB).
 __global__ void __launch_bounds__(256) k_integrate_3dx1d(const double* __restrict__ lm, int M, const double* __restrict__ mr,
                                                          int Q, const double* __restrict__ rz, int Z,
                                                          const double* __restrict__ dlnf, int F,
                                                          const double* __restrict__ dnum, double* __restrict__ numb) {
-    const uint32_t per_mq = (uint32_t)(Z - 1) * (uint32_t)F;
-    const uint32_t nchunk = (per_mq + blockDim.x - 1) / blockDim.x;
-    const int mq = (int)(blockIdx.x / nchunk);   // uniform: the block's chunks of one bin are consecutive
-    const int mm = mq / (Q - 1), qq = mq - mm * (Q - 1);
-    const uint32_t loc = (blockIdx.x - (uint32_t)mq * nchunk) * blockDim.x + threadIdx.x;
-    if (loc >= per_mq) return;
-    const int zz = (int)(loc / (uint32_t)F), ff = (int)(loc - (uint32_t)zz * (uint32_t)F);
-    const int64_t o = (int64_t)mq * per_mq + loc;
-    double dm = lm[mm + 1] - lm[mm];
-    double dmdq = dm * (mr[qq + 1] - mr[qq]);
-    double dmdqdz = dmdq * (rz[zz + 1] - rz[zz]);
-    double temp = 0.0;
+    const BinItem it = bin_item(Q, Z, F);
+    if (!it.live) return;
+    const int mm = it.mm, qq = it.qq, z0 = it.z0, ff = it.ff;
+    double v[4][BIN_ZC + 1];
+    bin_corners(dnum, it, Q, Z, F, v);
+    const double dm = lm[mm + 1] - lm[mm];
+    const double dmdq = dm * (mr[qq + 1] - mr[qq]);
+    double* o = numb + ((int64_t)it.mq * (Z - 1) + z0) * F + ff;
+    const double dl = dlnf[ff];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int k = 0; k < BIN_ZC; k++) {
+        if (z0 + k >= Z - 1) break;
+        const double dmdqdz = dmdq * (rz[z0 + k + 1] - rz[z0 + k]);
+        double temp = 0.0;   // mass, then ratio, then redshift: the reference's order
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int k = 0; k < 2; k++)
-                temp += dnum[((((int64_t)(mm + i) * Q) + (qq + j)) * Z + (zz + k)) * F + ff];
-    numb[o] = temp * dmdqdz * dlnf[ff] / 8.0;
+        for (int c = 0; c < 4; c++) {
+            temp += v[c][k];
+            temp += v[c][k + 1];
+        }
+        o[(int64_t)k * F] = temp * dmdqdz * dl / 8.0;
+    }
 }
 
 }  // namespace hd
@@ -726,9 +727,8 @@ extern "C" int hd_lifetime_2pwl(const double* norm_log10, const double* mtot, co
 extern "C" int hd_integrate_3dx1d(const double* log10_mtot, int M, const double* mrat, int Q, const double* redz, int Z,
                                   const double* dln_freq, int F, const double* dnum, double* numb, void* stream) {
     if (M < 2 || Q < 2 || Z < 2 || F < 1) return set_error(HD_ERR_ARG, "hd_integrate_3dx1d: bad sizes");
-    const int64_t per_mq = (int64_t)(Z - 1) * F;
-    const int64_t nblk = (int64_t)(M - 1) * (Q - 1) * cdiv(per_mq, 256);
-    if (per_mq > 0xffffffffll || nblk > 0x7fffffffll) return set_error(HD_ERR_SIZE, "hd_integrate_3dx1d: grid too large");
+    const int64_t nblk = bin_blocks(M, Q, Z, F);
+    if (nblk < 0) return set_error(HD_ERR_SIZE, "hd_integrate_3dx1d: grid too large");
     hipLaunchKernelGGL(k_integrate_3dx1d, dim3((unsigned)nblk), dim3(256), 0,
                        (hipStream_t)stream, log10_mtot, M, mrat, Q, redz, Z, dln_freq, F, dnum, numb);
     return check_launch("k_integrate_3dx1d");
