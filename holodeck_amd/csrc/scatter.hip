@@ -38,28 +38,32 @@ constexpr int CT_SLOT = 8;
 constexpr int CT_PIPE_LANES = 4;                        // lanes per vertex in the pipelined sweeps (a DPP quad)
 constexpr int CT_PIPE_ENT = CT_SLOT / CT_PIPE_LANES;    // entries per lane: lane k holds k, k + CT_PIPE_LANES, ...
 
+// (a thread sums the surpluses of a run of consecutive slots, one scan over the threads: 21 -> 12 us
+// at 7371 slots against a scan per 1024 of them)
 __global__ void __launch_bounds__(1024) k_ct_slots(int N, const int32_t* __restrict__ nptr,
                                                    const int32_t* __restrict__ lidx, int32_t* __restrict__ slot_ovf) {
-    __shared__ int32_t s_part[1024];
-    const int tid = threadIdx.x;
-    int32_t carry = 0;
-    for (int base = 0; base < N; base += 1024) {
-        const int t = base + tid;
-        int32_t d = (t < N) ? nptr[lidx[t] + 1] - nptr[lidx[t]] - CT_SLOT : 0;
-        d = d > 0 ? d : 0;
-        s_part[tid] = d;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            const int32_t v = (tid >= off) ? s_part[tid - off] : 0;
-            __syncthreads();
-            s_part[tid] += v;
-            __syncthreads();
-        }
-        if (t < N) slot_ovf[t] = carry + s_part[tid] - d;
-        carry += s_part[1023];
-        __syncthreads();
+    __shared__ int32_t s_wave[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int per = (N + 1023) / 1024, lo = min(tid * per, N), hi = min(lo + per, N);
+    auto surplus = [&](int t) { return max(nptr[lidx[t] + 1] - nptr[lidx[t]] - CT_SLOT, 0); };
+    int32_t sum = 0;
+#pragma unroll 8
+    for (int t = lo; t < hi; t++) sum += surplus(t);
+    int32_t inc = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t v = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += v;
     }
-    if (tid == 0) slot_ovf[N] = carry;
+    if (lane == 63) s_wave[w] = inc;
+    __syncthreads();
+    int32_t run = inc - sum;
+    for (int q = 0; q < w; q++) run += s_wave[q];
+    for (int t = lo; t < hi; t++) {
+        slot_ovf[t] = run;
+        run += surplus(t);
+    }
+    if (tid == 1023) slot_ovf[N] = run;
 }
 
 // Index of adjacency entry k of slot t in the padded layout.
@@ -73,43 +77,57 @@ __device__ __forceinline__ int64_t ct_entry(int64_t N, int t, int k, const int32
 // and per adjacency entry the neighbour, {ex, ey} and (ecap further on) {L^3, 1/L^3} -- the same
 // expressions in the same order as the sequential sweep evaluates them.  Pads: neighbour N and
 // {1, 1, 2, 1}, which with a constant of 1 and a zero value gives the term 1 - (2 - 1) = +0 through
-// the same operations, its q0 = 1 in the fast division's range.  Overflow entries beyond n_ovf are reported through *bad.
+// the same operations, its q0 = 1 in the fast division's range.  Eight lanes per slot (a lane per slot
+// waited for the one of 82 neighbours, a chain of that many loads and divisions: 42 -> 14 us).  Overflow entries beyond n_ovf are reported through *bad.
 __global__ void __launch_bounds__(256) k_ct_geom(int N, const double* __restrict__ pts, const int32_t* __restrict__ nptr,
                                                  const int32_t* __restrict__ nidx, const int32_t* __restrict__ lidx,
                                                  const int32_t* __restrict__ slot_ovf, int n_ovf,
                                                  int4* __restrict__ slot_i, double* __restrict__ slot_v,
                                                  int32_t* __restrict__ pe_q, double2* __restrict__ pe_geo,
                                                  int64_t ecap, int32_t* __restrict__ bad) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= N) return;
+    const int t = (blockIdx.x * blockDim.x + threadIdx.x) / CT_SLOT, lane8 = threadIdx.x % CT_SLOT;
+    if (t >= N) return;   // (whole groups of eight lanes)
     if (slot_ovf[N] > n_ovf) {
-        if (t == 0) atomicOr(bad, 1 << 20);
+        if (t == 0 && lane8 == 0) atomicOr(bad, 1 << 20);
         return;
     }
     const int p = lidx[t];
     const double px = pts[2 * p], py = pts[2 * p + 1];
     double Q0 = 0, Q1 = 0, Q3 = 0;
     const int deg = nptr[p + 1] - nptr[p];
-    for (int k = 0; k < deg; k++) {
-        const int q = nidx[nptr[p] + k];
-        const double ex = pts[2 * q] - px;
-        const double ey = pts[2 * q + 1] - py;
-        const double L = sqrt(ex * ex + ey * ey);
-        const double L3 = L * L * L;
-        Q0 += 4 * ex * ex / L3;
-        Q1 += 4 * ex * ey / L3;
-        Q3 += 4 * ey * ey / L3;
-        const int64_t e = ct_entry(N, t, k, slot_ovf);
-        pe_q[e] = q;
-        pe_geo[e] = make_double2(ex, ey);
-        pe_geo[ecap + e] = make_double2(L3, 1.0 / L3);
+    for (int k0 = 0; k0 < max(deg, CT_SLOT); k0 += CT_SLOT) {
+        const int k = k0 + lane8;
+        double c0 = 0, c1 = 0, c3 = 0;
+        if (k < deg) {
+            const int q = nidx[nptr[p] + k];
+            const double ex = pts[2 * q] - px;
+            const double ey = pts[2 * q + 1] - py;
+            const double L = sqrt(ex * ex + ey * ey);
+            const double L3 = L * L * L;
+            c0 = 4 * ex * ex / L3;
+            c1 = 4 * ex * ey / L3;
+            c3 = 4 * ey * ey / L3;
+            const int64_t e = ct_entry(N, t, k, slot_ovf);
+            pe_q[e] = q;
+            pe_geo[e] = make_double2(ex, ey);
+            pe_geo[ecap + e] = make_double2(L3, 1.0 / L3);
+        } else if (k < CT_SLOT) {
+            const int64_t e = ct_entry(N, t, k, slot_ovf);
+            pe_q[e] = N;
+            pe_geo[e] = make_double2(1.0, 1.0);
+            pe_geo[ecap + e] = make_double2(2.0, 1.0);
+        }
+#pragma unroll
+        for (int j = 0; j < CT_SLOT; j++) {   // in order
+            const double d0 = __shfl(c0, j, CT_SLOT), d1 = __shfl(c1, j, CT_SLOT), d3 = __shfl(c3, j, CT_SLOT);
+            if (k0 + j < deg) {
+                Q0 += d0;
+                Q1 += d1;
+                Q3 += d3;
+            }
+        }
     }
-    for (int k = deg; k < CT_SLOT; k++) {
-        const int64_t e = ct_entry(N, t, k, slot_ovf);
-        pe_q[e] = N;
-        pe_geo[e] = make_double2(1.0, 1.0);
-        pe_geo[ecap + e] = make_double2(2.0, 1.0);
-    }
+    if (lane8 != 0) return;
     const double Q2 = Q1;
     const double det = Q0 * Q3 - Q1 * Q2;
     slot_i[t] = make_int4(p, slot_ovf[t], slot_ovf[t + 1], 0);
@@ -1085,7 +1103,7 @@ extern "C" int hd_scatter(double* dens, int M, int Q, int Z, int G, const double
 
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, bad, 1);
     hipLaunchKernelGGL(k_ct_slots, dim3(1), dim3(1024), 0, st, N, nbr_ptr, levels_idx, slot_ovf);
-    hipLaunchKernelGGL(k_ct_geom, dim3((unsigned)cdiv(N, 256)), dim3(256), 0, st, N, pts, nbr_ptr, nbr_idx, levels_idx,
+    hipLaunchKernelGGL(k_ct_geom, dim3((unsigned)cdiv((int64_t)N * CT_SLOT, 256)), dim3(256), 0, st, N, pts, nbr_ptr, nbr_idx, levels_idx,
                        slot_ovf, n_ovf, slot_i, slot_v, pe_q, pe_geo, ecap, bad);
     hipLaunchKernelGGL(k_transpose_nz, dim3((unsigned)cdiv((int64_t)N * Z, 256)), dim3(256), 0, st, dens, N, Z, densT);
     hipLaunchKernelGGL(k_ct_fdiff, dim3((unsigned)cdiv((int64_t)N * Z, 256)), dim3(256), 0, st, densT, N, Z, ecap,
