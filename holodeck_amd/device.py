@@ -33,12 +33,15 @@ def ptr(t):
     return t.data_ptr()
 
 
-def to_dev(a, dtype=None):
+def to_dev(a, dtype=None, slots=False):
     """numpy array / scalar sequence / tensor -> contiguous device tensor (float64 default).
 
     Host arrays up to STAGE_MAX_BYTES are copied into a pinned staging ring and uploaded
     asynchronously on the current stream, so the host does not wait for the stream's earlier
-    work; larger arrays are copied synchronously (_Slots).  A tensor returned here is ready for work
+    work; larger arrays are copied by the runtime, or with ``slots`` through two pinned slots (_Slots):
+    faster for a caller that waits for the stream next, as the surrogate does, but the host then waits for
+    the stream's earlier kernels (a library with samples in flight on three streams, whose geometry is
+    uploaded between them: 222 samples/s against 135 through the slots).  A tensor returned here is ready for work
     on the current stream; another stream must wait for it (an event).
     """
     dev = require_device()
@@ -54,7 +57,9 @@ def to_dev(a, dtype=None):
     if host.numel() == 0:
         return torch.empty(host.shape, dtype=dtype, device=dev)
     staged = _staging().put(host) if host.numel() * host.element_size() <= STAGE_MAX_BYTES else None
-    if staged is None:                          # large: a synchronous copy
+    if staged is None:                          # large
+        if not slots:
+            return host.to(dev)
         out = torch.empty(host.shape, dtype=dtype, device=dev)
         if not _SLOTS.push(host.contiguous().view(-1).view(torch.uint8), out.view(-1).view(torch.uint8)):
             out.copy_(host)

@@ -148,8 +148,8 @@ class MLPSurrogate:
 
     def loss_and_grads(self, X01, Yn):
         """Device loss (MSE on standardised targets) and gradients for one batch; X01, Yn numpy or tensors."""
-        x = D.to_dev(np.asarray(X01, dtype=np.float32), dtype=torch.float32)
-        t = D.to_dev(np.asarray(Yn, dtype=np.float32), dtype=torch.float32)
+        x = D.to_dev(np.asarray(X01, dtype=np.float32), dtype=torch.float32, slots=True)
+        t = D.to_dev(np.asarray(Yn, dtype=np.float32), dtype=torch.float32, slots=True)
         step = _TrainStep.of(self, x, t, x.shape[0])
         if step is not None:
             loss = torch.zeros(1, dtype=torch.float32, device=x.device)
@@ -174,7 +174,7 @@ class MLPSurrogate:
         (continued training).
         """
         X = np.asarray(X, dtype=float)
-        Yn = D.to_dev(np.asarray(Y, dtype=float))
+        Yn = D.to_dev(np.asarray(Y, dtype=float), slots=True)
         if rescale:
             self.x_lo = X.min(axis=0) if x_lo is None else np.asarray(x_lo, float)
             self.x_hi = X.max(axis=0) if x_hi is None else np.asarray(x_hi, float)
@@ -269,7 +269,7 @@ class MLPSurrogate:
             else:
                 scale = D.to_dev(scale)
             for s0 in range(0, X.shape[0], chunk):
-                raw = X if one else D.to_dev(X[s0:s0 + chunk])
+                raw = X if one else D.to_dev(X[s0:s0 + chunk], slots=True)
                 y = D.empty((raw.shape[0], n_out))
                 _lib.call("hd_mlp_forward", C.addressof(net), None, D.ptr(raw), D.ptr(scale), y.shape[0], None,
                           D.ptr(y), D.stream_ptr())

@@ -43,3 +43,18 @@ def test_threads_on_their_own_streams(gpu):
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nbytes", [8, (256 << 10) + 8, (4 << 20) - 8, 4 << 20, (12 << 20) + 40])
+def test_uploads_through_the_slots(gpu, nbytes, monkeypatch):
+    """Only a caller that asks for the slots takes them: their upload waits for the stream's earlier
+    kernels, which callers with several streams in flight must not."""
+    from holodeck_amd import device as D
+    a = np.random.default_rng(nbytes).normal(size=nbytes // 8)
+    taken = []
+    push = D._SLOTS.push
+    monkeypatch.setattr(D._SLOTS, "push", lambda *args: taken.append(1) or push(*args))
+    assert np.array_equal(D.to_host(D.to_dev(a)), a) and not taken
+    assert np.array_equal(D.to_host(D.to_dev(a, slots=True)), a)
+    assert len(taken) == (1 if nbytes > D.STAGE_MAX_BYTES else 0)
