@@ -191,7 +191,7 @@ def surrogate_bench(n, judge_frac, seed=7):
         "judged": rep["n_judged"], "judged_median_dex_error": rep["median_dex_error"],
         "judged_p95_dex_error": rep["p95_dex_error"],
         "holdout_median_dex_error": float(net.meta['holdout_median_dex_error']),
-        "roofline": {"bound": "mfma", "kernel": "k_mlp_gemm (inference forward)", "achieved": tf,
+        "roofline": {"bound": "mfma", "kernel": "k_mlp_forward (inference)", "achieved": tf,
                      "peak": BF16_DENSE_PEAK_TFS, "unit": "TFLOP/s", "frac": tf / BF16_DENSE_PEAK_TFS,
                      "flops": flops, "gemm_ms": gemm_ms, "launches": gemm_n},
     }
