@@ -430,8 +430,8 @@ __global__ void __launch_bounds__(DBN_THREADS, 5) k_dbn_2pwl(EvoConsts K, const 
     const double age_universe = s_gage[n_interp - 1];
     // the step recorded per (kk, ff): the largest that brackets the target, as the reference's
     // last write over its in-order steps, above its left time's table interval (phase 2 need not search
-    // for it: 0.73 -> 0.66 ms with four divisions less per target); -1 none.  In LDS when it fits, else in redz_final as a 64-bit value + 1
-    // (0 none)
+    // for it: 0.73 -> 0.66 ms with four divisions less per target); -1 none.  In LDS when it
+    // fits, else in redz_final as a 64-bit value + 1 (0 none)
     const int nzf = Z * F;
     unsigned long long* rfg = (unsigned long long*)rf0;
     for (int p = tid; p < nzf; p += blockDim.x) {
@@ -441,7 +441,8 @@ __global__ void __launch_bounds__(DBN_THREADS, 5) k_dbn_2pwl(EvoConsts K, const 
     __syncthreads();
     // Only the steps whose bracket can hold a target are walked (sorted targets; 1.61 -> 0.73 ms at
     // 91x81x101 x 40): one evolution from 10^4 pc to the ISCO spans nine decades of separation, the
-    // targets of a PTA less than one and a half.  Below: a step's fr is its rest-frame frequency over 1 + z >= 1, so steps before the first
+    // targets of a PTA less than one and a half.  Below: a step's fr is its rest-frame frequency over
+    // 1 + z >= 1, so steps before the first
     // with s_frst[step + 1] >= fo[0] record nothing.  Above: once fl is past the last target (or the
     // time past the age of the universe) it stays there, as times and rest-frame frequencies grow; the
     // margins of 1e-3 and 1e-6 cover the rounding of time_left, at most a few 1e-16 of a total time

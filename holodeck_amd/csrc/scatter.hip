@@ -78,7 +78,8 @@ __device__ __forceinline__ int64_t ct_entry(int64_t N, int t, int k, const int32
 // expressions in the same order as the sequential sweep evaluates them.  Pads: neighbour N and
 // {1, 1, 2, 1}, which with a constant of 1 and a zero value gives the term 1 - (2 - 1) = +0 through
 // the same operations, its q0 = 1 in the fast division's range.  Eight lanes per slot (a lane per slot
-// waited for the one of 82 neighbours, a chain of that many loads and divisions: 42 -> 14 us).  Overflow entries beyond n_ovf are reported through *bad.
+// waited for the one of 82 neighbours, a chain of that many loads and divisions: 42 -> 14 us).
+// Overflow entries beyond n_ovf are reported through *bad.
 __global__ void __launch_bounds__(256) k_ct_geom(int N, const double* __restrict__ pts, const int32_t* __restrict__ nptr,
                                                  const int32_t* __restrict__ nidx, const int32_t* __restrict__ lidx,
                                                  const int32_t* __restrict__ slot_ovf, int n_ovf,
