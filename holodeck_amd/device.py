@@ -156,8 +156,10 @@ class _Slots:
         return True
 
     def fetch(self, src, dst):
-        """src: 1-D uint8 device tensor, as the current stream leaves it; dst: host tensor of its size.
-        False (nothing done) when another caller holds the slots."""
+        """src: 1-D uint8 device tensor, as its device's current stream leaves it (where the copies run, so
+        where their events belong); dst: host tensor of its size.  False (nothing done) when another
+        caller holds the slots."""
+        stream = torch.cuda.current_stream(src.device)
         if not self._take():
             return False
         flying = None
@@ -167,7 +169,7 @@ class _Slots:
                 slot = self.slots[k & 1][:part.numel()]
                 slot.copy_(part, non_blocking=True)
                 ev = torch.cuda.Event()
-                ev.record()
+                ev.record(stream)
                 if flying is not None:
                     self._land(*flying)
                 flying = (dst[s0:s0 + SLOT_BYTES], slot, ev)
@@ -183,8 +185,9 @@ class _Slots:
         dst.copy_(slot)
 
     def push(self, src, dst):
-        """src: 1-D uint8 host tensor; dst: device tensor of its size, written on the current stream
-        before this returns.  False (nothing done) when another caller holds the slots."""
+        """src: 1-D uint8 host tensor; dst: device tensor of its size, written on its device's current
+        stream before this returns.  False (nothing done) when another caller holds the slots."""
+        stream = torch.cuda.current_stream(dst.device)
         if not self._take():
             return False
         busy = [None, None]
@@ -197,7 +200,7 @@ class _Slots:
                 slot.copy_(part)
                 dst[s0:s0 + SLOT_BYTES].copy_(slot, non_blocking=True)
                 busy[k & 1] = torch.cuda.Event()
-                busy[k & 1].record()
+                busy[k & 1].record(stream)
             for ev in busy:
                 if ev is not None:
                     ev.synchronize()
@@ -210,8 +213,8 @@ _SLOTS = _Slots()
 
 
 def to_host(t, out=None):
-    """Host numpy copy of a tensor (waits for the current stream); into the contiguous array ``out`` if
-    given."""
+    """Host numpy copy of a tensor (waits for its device's current stream); into the contiguous array
+    ``out`` if given."""
     t = t.detach()
     if not t.is_cuda or t.numel() * t.element_size() < DOWNLOAD_MIN_BYTES:
         if out is None:

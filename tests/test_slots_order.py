@@ -1,0 +1,115 @@
+"""The pinned slots' order of copies and waits, on a model of asynchronous copies (CPU): a copy between a
+slot and a device tensor waits in the queue of that tensor's device and is made when something waits for
+the queue.  What the host reads before that is what the slot held before."""
+import collections
+
+import pytest
+import torch
+
+from holodeck_amd import device as D
+
+SLOT = 4 << 10
+
+
+class Sim(torch.Tensor):
+    """A tensor with a place of its own: 'slot', or a device index."""
+    place = None
+
+    @classmethod
+    def at(cls, t, place):
+        t = t.as_subclass(cls)
+        t.place = place
+        return t
+
+    @property
+    def device(self):
+        return torch.device("cuda", self.place) if isinstance(self.place, int) else torch.device("cpu")
+
+    def __getitem__(self, k):
+        return Sim.at(self.as_subclass(torch.Tensor)[k], self.place)
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        if func is not torch.Tensor.copy_:
+            return super().__torch_function__(func, types, args, kwargs or {})
+        dst, src = args
+        place = [t.place for t in (dst, src) if isinstance(t, Sim) and isinstance(t.place, int)]
+        d, s = dst.as_subclass(torch.Tensor), src.as_subclass(torch.Tensor)
+        if place:
+            assert kwargs == {"non_blocking": True}
+            World.queue[place[0]].append(lambda: d.copy_(s))
+        else:
+            d.copy_(s)
+        return dst
+
+
+class World:
+    """One stream per device; device 0 is the current one."""
+    queue = collections.defaultdict(list)
+    interrupt = 0      # raise at this wait (1: the first)
+
+    @classmethod
+    def drain(cls, place, upto=None):
+        q = cls.queue[place]
+        while q and (upto is None or upto > 0):
+            q.pop(0)()
+            upto = None if upto is None else upto - 1
+
+    class Stream:
+        def __init__(self, place):
+            self.place = place
+
+        def synchronize(self):
+            World.drain(self.place)
+
+    class Event:
+        def record(self, stream=None):
+            self.place = 0 if stream is None else stream.place
+            self.upto = list(World.queue[self.place])
+
+        def synchronize(self):
+            World.interrupt -= 1
+            if World.interrupt == 0:
+                raise KeyboardInterrupt
+            for op in self.upto:
+                if op in World.queue[self.place]:
+                    World.queue[self.place].remove(op)
+                    op()
+
+
+@pytest.fixture
+def slots(monkeypatch):
+    World.queue.clear()
+    World.interrupt = 0
+    real_empty = torch.empty
+
+    def empty(*shape, **kw):
+        if not kw.pop("pin_memory", False):
+            return real_empty(*shape, **kw)
+        return Sim.at(real_empty(*shape, **kw).fill_(255), "slot")
+
+    def current_stream(device=None):
+        index = getattr(device, "index", device)
+        return World.Stream(0 if index is None else index)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    monkeypatch.setattr(torch.cuda, "Event", World.Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    monkeypatch.setattr(D, "SLOT_BYTES", SLOT)
+    return D._Slots()
+
+
+def _data(n, seed):
+    return torch.randint(0, 200, (n,), dtype=torch.uint8, generator=torch.Generator().manual_seed(seed))
+
+
+@pytest.mark.parametrize("place", [0, 1])
+@pytest.mark.parametrize("n", [1, SLOT - 1, SLOT, SLOT + 1, 5 * SLOT + 7])
+def test_copies_wait_for_the_tensors_own_device(slots, place, n):
+    a = _data(n, n)
+    got = torch.zeros(n, dtype=torch.uint8)
+    assert slots.fetch(Sim.at(a.clone(), place), got)
+    assert torch.equal(got, a)
+    put = torch.zeros(n, dtype=torch.uint8)
+    assert slots.push(a.clone(), Sim.at(put, place))
+    assert torch.equal(put, a)
