@@ -138,7 +138,9 @@ SLOT_BYTES = 4 << 20
 class _Slots:
     """Two pinned slots through which larger arrays pass between host and device: one is in flight by DMA
     (56 GB/s measured; the runtime's pageable copies reach 4) while the host's threads copy the other
-    from or to its place.  One caller at a time; others meanwhile take the runtime's own copy."""
+    from or to its place.  One caller at a time; others meanwhile take the runtime's own copy.  After an
+    exception (an interrupted wait) a copy may still be in flight in a slot: the slots are given up, and
+    torch's host allocator hands their memory out again only when those copies are done."""
 
     def __init__(self):
         self.lock = threading.Lock()
@@ -175,6 +177,9 @@ class _Slots:
                 flying = (dst[s0:s0 + SLOT_BYTES], slot, ev)
             if flying is not None:
                 self._land(*flying)
+        except BaseException:
+            self.slots = None
+            raise
         finally:
             self.lock.release()
         return True
@@ -204,6 +209,9 @@ class _Slots:
             for ev in busy:
                 if ev is not None:
                     ev.synchronize()
+        except BaseException:
+            self.slots = None
+            raise
         finally:
             self.lock.release()
         return True

@@ -113,3 +113,41 @@ def test_copies_wait_for_the_tensors_own_device(slots, place, n):
     put = torch.zeros(n, dtype=torch.uint8)
     assert slots.push(a.clone(), Sim.at(put, place))
     assert torch.equal(put, a)
+
+
+@pytest.mark.parametrize("way", ["fetch", "push"])
+@pytest.mark.parametrize("wait", [1, 2])
+def test_an_interrupted_copy_keeps_its_slots_to_itself(slots, way, wait):
+    """The copies still in flight when a wait is interrupted run after the next caller has filled its slots."""
+    a, b = _data(6 * SLOT, 1), _data(2 * SLOT, 2)
+    put = torch.zeros_like(a)
+    World.interrupt = wait
+    with pytest.raises(KeyboardInterrupt):
+        if way == "fetch":
+            slots.fetch(Sim.at(a.clone(), 1), torch.zeros_like(a))
+        else:
+            slots.push(a.clone(), Sim.at(put, 1))
+    late = list(World.queue[1])
+    assert late
+    World.queue[1].clear()
+    World.interrupt = 0
+    got = torch.zeros_like(b)
+    land = D._Slots._land
+
+    def after_the_late_ones(dst, slot, ev):
+        ev.synchronize()
+        while late:
+            late.pop(0)()
+        dst.copy_(slot)
+
+    slots._land = after_the_late_ones if way == "fetch" else land
+    assert slots.fetch(Sim.at(b.clone(), 0), got)
+    assert torch.equal(got, b)
+    if way == "push":      # what was queued before the interruption still holds its own data
+        n = len(late)
+        while late:
+            late.pop(0)()
+        done = [k for k in range(6) if put[k * SLOT:(k + 1) * SLOT].any()]
+        assert len(done) >= n
+        for k in done:
+            assert torch.equal(put[k * SLOT:(k + 1) * SLOT], a[k * SLOT:(k + 1) * SLOT])
