@@ -152,6 +152,9 @@ class _Slots:
         if self.slots is None:
             try:
                 self.slots = [torch.empty(SLOT_BYTES, dtype=torch.uint8, pin_memory=True) for _ in range(2)]
+            except RuntimeError:    # no pinned memory: the runtime's own copy needs none
+                self.lock.release()
+                return False
             except BaseException:
                 self.lock.release()
                 raise
@@ -160,7 +163,7 @@ class _Slots:
     def fetch(self, src, dst):
         """src: 1-D uint8 device tensor, as its device's current stream leaves it (where the copies run, so
         where their events belong); dst: host tensor of its size.  False (nothing done) when another
-        caller holds the slots."""
+        caller holds the slots or none can be had."""
         stream = torch.cuda.current_stream(src.device)
         if not self._take():
             return False
@@ -191,7 +194,7 @@ class _Slots:
 
     def push(self, src, dst):
         """src: 1-D uint8 host tensor; dst: device tensor of its size, written on its device's current
-        stream before this returns.  False (nothing done) when another caller holds the slots."""
+        stream before this returns.  False (nothing done) when another caller holds the slots or none can be had."""
         stream = torch.cuda.current_stream(dst.device)
         if not self._take():
             return False

@@ -151,3 +151,13 @@ def test_an_interrupted_copy_keeps_its_slots_to_itself(slots, way, wait):
         assert len(done) >= n
         for k in done:
             assert torch.equal(put[k * SLOT:(k + 1) * SLOT], a[k * SLOT:(k + 1) * SLOT])
+
+
+def test_without_pinned_memory_the_runtime_copies(slots, monkeypatch):
+    """No pinned memory to be had: the caller is told to take the runtime's own copy, each time."""
+    def none_left(*shape, **kw):
+        raise torch.cuda.OutOfMemoryError("HIP out of memory")
+    monkeypatch.setattr(torch, "empty", none_left)
+    a = _data(9, 3)
+    for _ in range(2):
+        assert not slots.fetch(Sim.at(a.clone(), 0), a) and not slots.push(a, Sim.at(a.clone(), 0))
