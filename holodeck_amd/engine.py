@@ -213,10 +213,23 @@ def eccen_number(ndens, mtot_log10_d, mrat_d, redz_d, dcom_d, gwfobs_d, sepa_d, 
     return lam, hv
 
 
+def _eccen_chunk_ws_bytes(B, F, R):
+    """Realization workspace that eccen_harm_chunk counts: records and sparse axes of 512-bin tiles,
+    totals of 8-tile items, 8 merge groups.  A definition of its own, not the present workspace's size:
+    the chunks decide the draws of a seed, which must not move with the layout of a kernel."""
+    def up(n):
+        return (n + 255) & ~255
+    tiles = -(-B // 512)
+    items = F * -(-tiles // 8)
+    return (up(4 * B) + up(48 * 513 * F * tiles) + up(4 * 513 * F * tiles) + up(12 * F * tiles) +
+            3 * up(8 * 512 * F * tiles) + up(8 * items * R) + up(8 * 8 * F * R + 1024) + 2 * up(4 * items) +
+            up(4 * F * tiles) + 512)
+
+
 def eccen_harm_chunk(B, F, nharms, nreals):
     """Harmonics per chunk of the discrete variant: Poisson means, strain factors and the
-    realization workspace of one chunk within ECCEN_WS_COLUMNS_BYTES."""
-    per_col = 16 * B + _lib.size("hd_realize_workspace_size", B, F, int(nreals), 0, 0) / max(F, 1)
+    realization workspace of one chunk within about ECCEN_WS_COLUMNS_BYTES."""
+    per_col = 16 * B + _eccen_chunk_ws_bytes(B, F, int(nreals)) / max(F, 1)
     return int(max(1, min(nharms, ECCEN_WS_COLUMNS_BYTES // (per_col * F))))
 
 
