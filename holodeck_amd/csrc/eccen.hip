@@ -103,7 +103,9 @@ __device__ __noinline__ void bessel_pair(int lo, double x, double& j_lo, double&
         }
     };
     double norm;
-    if (a <= ECC_LOW_ORDER || x < 1e-12) {   // (tiny arguments: the terms grow by 1e12 a step and more)
+    // (tiny arguments, for their order or at all: a term is 2 k / x times the one before it.  From
+    // 4e-15 (a + 2) on that is below 2e15, and four steps from 1e240 stay below 2e301)
+    if (a <= ECC_LOW_ORDER || x < 1e-12 || x < 4e-15 * (double)(a + 2)) {
         const double big = fmax((double)(a + 2), x);
         const int m = 2 * ((int)(big + sqrt(160.0 * big) + 10.0) / 2);
         k = (double)m;
