@@ -357,8 +357,9 @@ int realize_merge_launch(const double* h2fdf, const double* par, const int64_t* 
 
 // Bins per chunk of given counts: about RZ_WAVES waves over the columns, at least RZ_MIN_CHUNK
 // bins (a chunk's partial costs as much as a few bins) and at most RZ_MAX_CHUNKS chunks (the merge
-// walks them).
+// walks them).  The workspace query asks before the sizes are checked: empty ones get the least chunk.
 static int counts_chunk_bins(int64_t B, int F, int R) {
+    if (B < 1 || F < 1 || R < 1) return RZ_MIN_CHUNK;
     const int64_t waves = cdiv((int64_t)F * R, 64);
     int64_t nch = cdiv(RZ_WAVES, waves);
     nch = std::min(nch, std::min((int64_t)RZ_MAX_CHUNKS, cdiv(B, RZ_MIN_CHUNK)));
