@@ -116,6 +116,7 @@ struct GapArgs {
     int64_t B;
     int F, R, L, flags, npar, ntiles, nchunks, mode, cap;
     int tpc;                // tiles per chunk
+    int px;                 // draw workgroups of an item along x, bs realizations each; the rest along y
     double thresh, tau;
     uint64_t seed;
     DRec* drec;             // (F, ntiles, GZ_REC)
@@ -1127,12 +1128,14 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     uint32_t* tab = (uint32_t*)gz_lds;   // A.cap 8-byte slots: per record n high words, then n low words
     double* scum = gz_lds + A.cap;     // GZ_TILE doubles
     BRec* brec = (BRec*)(scum + GZ_TILE);   // GZ_BATCH_REC staged record headers
-    const int item = A.plan[blockIdx.x];   // heaviest items first
+    const int item = A.plan[blockIdx.x / A.px];   // heaviest items first
     const int f = item / A.nchunks;
     const int chunk = item - f * A.nchunks;
     const int tid = threadIdx.x, lane = tid & 63;
     const int bs = blockDim.x;
     const int F = A.F, R = A.R, L = A.L;
+    const int rbase = (int)(blockIdx.y * A.px + blockIdx.x % A.px) * bs;   // this workgroup's realizations
+    if (rbase >= R) return;
     const int t0 = chunk * A.tpc;
     const int t1 = min(t0 + A.tpc, A.ntiles);
     const int64_t pstride = (int64_t)F * A.ntiles * GZ_TILE;
@@ -1144,185 +1147,183 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
     }
     __syncthreads();
 
-    for (int rbase = 0; rbase < R; rbase += bs) {
-        const int r = rbase + tid;
-        const bool active = r < R;
-        Acc<MODE, LM, NP> acc;
-        acc.init();
-        for (int tile = t0; tile < t1; tile++) {
-            const int64_t ft = (int64_t)f * A.ntiles + tile;
-            const int64_t reg = ft * GZ_TILE;
-            const int64_t rreg = ft * GZ_REC;
-            const int nd = s_cnt[tile - t0][0], ns = s_cnt[tile - t0][1];
-            const int nrec = nd + (ns > 0 ? 1 : 0);
-            // the realization's stream for this tile: records in order take one word each
-            // (two when the 32-bit draw is open), then the sparse points two words each
-            Xo128 rs;
-            rs.seed(philox4x32_10(U4{(uint32_t)tile, (uint32_t)f, (uint32_t)r, 6u << 16}, k0, k1));
-            int c = 0, base = 0;   // base: where the batch's tables start among the tile's
-            while (c < nrec) {
-                // batch [c, c1): consecutive records whose windows fit the table, at most
-                // GZ_BATCH_REC.  The record this thread stages is loaded with the record ends: its
-                // place does not depend on where the batch ends
-                const DRec mine = A.drec[rreg + min(c + tid, nrec - 1)];
-                const int e0 = A.rec_end[rreg + min(c + lane, nrec - 1)];
-                const int e1 = A.rec_end[rreg + min(c + 64 + lane, nrec - 1)];
-                const int limit = base + A.cap;
-                int c1 = c + __popcll(__ballot(c + lane < nrec && e0 <= limit)) +
-                         __popcll(__ballot(c + 64 + lane < nrec && e1 <= limit));
-                c1 = max(c1, c + 1);   // every window fits alone (n <= cap); keeps progress unconditional
-                const int base_next = (c1 - c <= 64) ? __builtin_amdgcn_readlane(e0, c1 - c - 1)
-                                                     : __builtin_amdgcn_readlane(e1, c1 - c - 65);
-                if (tid == 0) {
-                    s_next = 0;
-                    s_nlarge = 0;
-                    s_nrow = 0;
-                    s_nshort = 0;
-                    s_lsum = 0;
+    const int r = rbase + tid;
+    const bool active = r < R;
+    Acc<MODE, LM, NP> acc;
+    acc.init();
+    for (int tile = t0; tile < t1; tile++) {
+        const int64_t ft = (int64_t)f * A.ntiles + tile;
+        const int64_t reg = ft * GZ_TILE;
+        const int64_t rreg = ft * GZ_REC;
+        const int nd = s_cnt[tile - t0][0], ns = s_cnt[tile - t0][1];
+        const int nrec = nd + (ns > 0 ? 1 : 0);
+        // the realization's stream for this tile: records in order take one word each
+        // (two when the 32-bit draw is open), then the sparse points two words each
+        Xo128 rs;
+        rs.seed(philox4x32_10(U4{(uint32_t)tile, (uint32_t)f, (uint32_t)r, 6u << 16}, k0, k1));
+        int c = 0, base = 0;   // base: where the batch's tables start among the tile's
+        while (c < nrec) {
+            // batch [c, c1): consecutive records whose windows fit the table, at most
+            // GZ_BATCH_REC.  The record this thread stages is loaded with the record ends: its
+            // place does not depend on where the batch ends
+            const DRec mine = A.drec[rreg + min(c + tid, nrec - 1)];
+            const int e0 = A.rec_end[rreg + min(c + lane, nrec - 1)];
+            const int e1 = A.rec_end[rreg + min(c + 64 + lane, nrec - 1)];
+            const int limit = base + A.cap;
+            int c1 = c + __popcll(__ballot(c + lane < nrec && e0 <= limit)) +
+                     __popcll(__ballot(c + 64 + lane < nrec && e1 <= limit));
+            c1 = max(c1, c + 1);   // every window fits alone (n <= cap); keeps progress unconditional
+            const int base_next = (c1 - c <= 64) ? __builtin_amdgcn_readlane(e0, c1 - c - 1)
+                                                 : __builtin_amdgcn_readlane(e1, c1 - c - 65);
+            if (tid == 0) {
+                s_next = 0;
+                s_nlarge = 0;
+                s_nrow = 0;
+                s_nshort = 0;
+                s_lsum = 0;
+            }
+            __syncthreads();   // the previous batch's draws are done with tab / scum
+            // one thread per record of the batch stages its header and lists its table as
+            // short (at most GZ_SEQ_MAX counts summed) or long
+            if (c + tid < c1) {
+                const DRec& rec = mine;
+                brec[tid] = gz_header(rec.lam, rec.p0, rec.kt, rec.n, rec.off - base, rec.kb);
+                const int nb = rec.kt + rec.n - rec.kb;
+                if (rec.n > 0 && nb <= GZ_SEQ_MAX) s_short[atomicAdd(&s_nshort, 1)] = tid;
+                else if (rec.n > 0 && nb <= HD_GZ_ROW_MAX) s_row[atomicAdd(&s_nrow, 1)] = tid;
+                else if (rec.n > 0) {
+                    s_large[atomicAdd(&s_nlarge, 1)] = tid;
+                    atomicAdd(&s_lsum, nb);
                 }
-                __syncthreads();   // the previous batch's draws are done with tab / scum
-                // one thread per record of the batch stages its header and lists its table as
-                // short (at most GZ_SEQ_MAX counts summed) or long
-                if (c + tid < c1) {
-                    const DRec& rec = mine;
-                    brec[tid] = gz_header(rec.lam, rec.p0, rec.kt, rec.n, rec.off - base, rec.kb);
-                    const int nb = rec.kt + rec.n - rec.kb;
-                    if (rec.n > 0 && nb <= GZ_SEQ_MAX) s_short[atomicAdd(&s_nshort, 1)] = tid;
-                    else if (rec.n > 0 && nb <= HD_GZ_ROW_MAX) s_row[atomicAdd(&s_nrow, 1)] = tid;
-                    else if (rec.n > 0) {
-                        s_large[atomicAdd(&s_nlarge, 1)] = tid;
-                        atomicAdd(&s_lsum, nb);
-                    }
+            }
+            __syncthreads();
+            // build items handed out to the waves one at a time, the longest serial work
+            // first: long tables (a wave each), then mid-size tables four at a time (a
+            // 16-lane row each), then groups of 64 short tables (a lane each, one
+            // sequential pass), so that every lane a build occupies has work
+            {
+                int nl = s_nlarge;
+                const int nr = s_nrow, nsh = s_nshort;
+                const int parts = gz_parts(nl, s_lsum);
+                if (parts > 1) {   // few long tables: cut so that each wave builds a part
+                    const int wv = tid >> 6;
+                    const BRec* rec = brec + s_large[min(wv / parts, nl - 1)];
+                    const int part = wv % parts, nb = rec->kt + rec->n - rec->kb;
+                    const bool on = wv < nl * parts;
+                    GzPart P;
+                    gz_lds_u32* hi = (gz_lds_u32*)(tab + 2 * rec->off);
+                    if (on)
+                        P = gz_part_sum((gz_lrec)rec, hi, gz_part_edge(nb, part, parts), gz_part_edge(nb, part + 1, parts),
+                                        lane, s_part[wv]);
+                    __syncthreads();
+                    if (on) gz_part_write((gz_lrec)rec, hi, P, part, s_part[wv - part]);
+                    nl = 0;
                 }
-                __syncthreads();
-                // build items handed out to the waves one at a time, the longest serial work
-                // first: long tables (a wave each), then mid-size tables four at a time (a
-                // 16-lane row each), then groups of 64 short tables (a lane each, one
-                // sequential pass), so that every lane a build occupies has work
-                {
-                    int nl = s_nlarge;
-                    const int nr = s_nrow, nsh = s_nshort;
-                    const int parts = gz_parts(nl, s_lsum);
-                    if (parts > 1) {   // few long tables: cut so that each wave builds a part
-                        const int wv = tid >> 6;
-                        const BRec* rec = brec + s_large[min(wv / parts, nl - 1)];
-                        const int part = wv % parts, nb = rec->kt + rec->n - rec->kb;
-                        const bool on = wv < nl * parts;
-                        GzPart P;
-                        gz_lds_u32* hi = (gz_lds_u32*)(tab + 2 * rec->off);
-                        if (on)
-                            P = gz_part_sum((gz_lrec)rec, hi, gz_part_edge(nb, part, parts), gz_part_edge(nb, part + 1, parts),
-                                            lane, s_part[wv]);
-                        __syncthreads();
-                        if (on) gz_part_write((gz_lrec)rec, hi, P, part, s_part[wv - part]);
-                        nl = 0;
-                    }
-                    const int nrg = (nr + 3) >> 2, nsg = (nsh + 63) >> 6;
-                    for (;;) {
-                        int w = 0;
-                        if (lane == 0) w = atomicAdd(&s_next, 1);
-                        w = __shfl(w, 0, 64);
-                        if (w >= nl + nrg + nsg) break;
-                        if (w < nl) {
-                            const BRec* rec = brec + s_large[w];
-                            gz_build<64>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), true, lane);
-                        } else if (w < nl + nrg) {
-                            const int k = (w - nl) * 4 + (lane >> 4);
-                            const bool on = k < nr;
-                            const BRec* rec = brec + s_row[on ? k : 0];
-                            gz_build<16>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), on, lane & 15);
-                        } else {
-                            const int k = (w - nl - nrg) * 64 + lane;
-                            if (k < nsh) {
-                                const BRec* rec = brec + s_short[k];
-                                gz_build_seq((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kt, rec->n, rec->p0);
-                            }
+                const int nrg = (nr + 3) >> 2, nsg = (nsh + 63) >> 6;
+                for (;;) {
+                    int w = 0;
+                    if (lane == 0) w = atomicAdd(&s_next, 1);
+                    w = __shfl(w, 0, 64);
+                    if (w >= nl + nrg + nsg) break;
+                    if (w < nl) {
+                        const BRec* rec = brec + s_large[w];
+                        gz_build<64>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), true, lane);
+                    } else if (w < nl + nrg) {
+                        const int k = (w - nl) * 4 + (lane >> 4);
+                        const bool on = k < nr;
+                        const BRec* rec = brec + s_row[on ? k : 0];
+                        gz_build<16>((gz_lrec)rec, (gz_lds_u32*)(tab + 2 * rec->off), on, lane & 15);
+                    } else {
+                        const int k = (w - nl - nrg) * 64 + lane;
+                        if (k < nsh) {
+                            const BRec* rec = brec + s_short[k];
+                            gz_build_seq((gz_lds_u32*)(tab + 2 * rec->off), rec->lam, rec->kt, rec->n, rec->p0);
                         }
                     }
                 }
-                if (c1 == nrec && ns > 0)
-                    for (int j = tid; j < ns; j += bs) scum[j] = A.s_cum[reg + j];
-                __syncthreads();
-                if (active) {
-                    // dense records of the batch (one control path, so the running list needs no
-                    // copies between branches), then the tile's sparse pseudo-record if it is here
-                    // (records in pairs, their searches interleaved; n = 0: no table, drawn by k_gz_big)
-                    // the records' fields are the same for every lane: read through the constant
-                    // address space (scalar loads into SGPRs, no VALU moves); the staged LDS copy
-                    // serves the builds and the rare tail walk
-                    // the next pair's records are loaded before the current pair is drawn
-                    const int cd = min(c1, nd);
-                    const DRec* rec = A.drec + rreg;
-                    {
-                        int pairs_to = c;   // records before this are drawn in pairs
-                        for (int i = c; i < cd; i += 2) {
-                            if (i >= pairs_to && i + 4 <= cd) {
-                                GzDraw d[4];
-                                GzTab t[4];
-                                int k[4], shortest = 1;
+            }
+            if (c1 == nrec && ns > 0)
+                for (int j = tid; j < ns; j += bs) scum[j] = A.s_cum[reg + j];
+            __syncthreads();
+            if (active) {
+                // dense records of the batch (one control path, so the running list needs no
+                // copies between branches), then the tile's sparse pseudo-record if it is here
+                // (records in pairs, their searches interleaved; n = 0: no table, drawn by k_gz_big)
+                // the records' fields are the same for every lane: read through the constant
+                // address space (scalar loads into SGPRs, no VALU moves); the staged LDS copy
+                // serves the builds and the rare tail walk
+                // the next pair's records are loaded before the current pair is drawn
+                const int cd = min(c1, nd);
+                const DRec* rec = A.drec + rreg;
+                {
+                    int pairs_to = c;   // records before this are drawn in pairs
+                    for (int i = c; i < cd; i += 2) {
+                        if (i >= pairs_to && i + 4 <= cd) {
+                            GzDraw d[4];
+                            GzTab t[4];
+                            int k[4], shortest = 1;
+#pragma unroll
+                            for (int q = 0; q < 4; q++) {
+                                d[q] = gz_load_draw(rec + i + q);
+                                t[q] = gz_tab_rec(tab, d[q], base, brec + (i + q - c), true);
+                                shortest = min(shortest, d[q].n);
+                            }
+                            if (shortest > 0 && gz_draw4(t, rs, k)) {
+                                const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
 #pragma unroll
                                 for (int q = 0; q < 4; q++) {
-                                    d[q] = gz_load_draw(rec + i + q);
-                                    t[q] = gz_tab_rec(tab, d[q], base, brec + (i + q - c), true);
-                                    shortest = min(shortest, d[q].n);
+                                    acc.add((double)k[q], d[q].h, d[q].word, par + q, pstride, A.npar, L);
+                                    if (REC) gz_record(A, d[q].word, f, r, (double)k[q], false);
                                 }
-                                if (shortest > 0 && gz_draw4(t, rs, k)) {
-                                    const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
-#pragma unroll
-                                    for (int q = 0; q < 4; q++) {
-                                        acc.add((double)k[q], d[q].h, d[q].word, par + q, pstride, A.npar, L);
-                                        if (REC) gz_record(A, d[q].word, f, r, (double)k[q], false);
-                                    }
-                                    i += 2;
-                                    continue;
-                                }
-                                pairs_to = i + 4;
+                                i += 2;
+                                continue;
                             }
-                            const bool hb = i + 1 < cd;
-                            const GzDraw ra = gz_load_draw(rec + i), rb = gz_load_draw(rec + (hb ? i + 1 : i));
-                            const GzTab ta = gz_tab_rec(tab, ra, base, brec + (i - c), true);
-                            const GzTab tb = gz_tab_rec(tab, rb, base, brec + (hb ? i + 1 - c : i - c), hb);
-                            int ka, kb;
-                            gz_draw2(ta, tb, rs, ka, kb);
-                            const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
-                            if (ta.n > 0) acc.add((double)ka, ra.h, ra.word, par, pstride, A.npar, L);
-                            if (tb.n > 0) acc.add((double)kb, rb.h, rb.word, par + 1, pstride, A.npar, L);
-                            if (REC) {
-                                if (ta.n > 0) gz_record(A, ra.word, f, r, (double)ka, false);
-                                if (tb.n > 0) gz_record(A, rb.word, f, r, (double)kb, false);
-                            }
+                            pairs_to = i + 4;
                         }
-                    }
-                    for (int i = max(c, nd); i < c1; i++) {
-                        const BRec* rec = brec + (i - c);
-                        {
-                            // sparse bins: Poisson process on the tile's cumulative-lambda axis; the
-                            // point count from its table (it always fits: lambda < 512), the
-                            // positions uniform on the axis (53-bit uniforms)
-                            const double Lam = scum[ns - 1];
-                            const int np = gz_draw1(gz_tab(tab, rec, true), rs);
-                            for (int q = 0; q < np; q++) {
-                                const uint32_t w0 = rs.next();
-                                const double xq = u53(w0, rs.next()) * Lam;
-                                int lo = 0, hi = ns - 1;
-                                while (lo < hi) {   // first j with scum[j] > xq
-                                    const int mid = (lo + hi) >> 1;
-                                    if (scum[mid] > xq) hi = mid;
-                                    else lo = mid + 1;
-                                }
-                                acc.add(1.0, A.s_h[reg + lo], A.s_word[reg + lo], A.sp_par + reg + lo, pstride, A.npar,
-                                        L);
-                                if (REC) gz_record(A, A.s_word[reg + lo], f, r, 1.0, true);
-                            }
+                        const bool hb = i + 1 < cd;
+                        const GzDraw ra = gz_load_draw(rec + i), rb = gz_load_draw(rec + (hb ? i + 1 : i));
+                        const GzTab ta = gz_tab_rec(tab, ra, base, brec + (i - c), true);
+                        const GzTab tb = gz_tab_rec(tab, rb, base, brec + (hb ? i + 1 - c : i - c), hb);
+                        int ka, kb;
+                        gz_draw2(ta, tb, rs, ka, kb);
+                        const gz_cpar par = (gz_cpar)(A.d_par + reg + i);
+                        if (ta.n > 0) acc.add((double)ka, ra.h, ra.word, par, pstride, A.npar, L);
+                        if (tb.n > 0) acc.add((double)kb, rb.h, rb.word, par + 1, pstride, A.npar, L);
+                        if (REC) {
+                            if (ta.n > 0) gz_record(A, ra.word, f, r, (double)ka, false);
+                            if (tb.n > 0) gz_record(A, rb.word, f, r, (double)kb, false);
                         }
                     }
                 }
-                c = c1;
-                base = base_next;
+                for (int i = max(c, nd); i < c1; i++) {
+                    const BRec* rec = brec + (i - c);
+                    {
+                        // sparse bins: Poisson process on the tile's cumulative-lambda axis; the
+                        // point count from its table (it always fits: lambda < 512), the
+                        // positions uniform on the axis (53-bit uniforms)
+                        const double Lam = scum[ns - 1];
+                        const int np = gz_draw1(gz_tab(tab, rec, true), rs);
+                        for (int q = 0; q < np; q++) {
+                            const uint32_t w0 = rs.next();
+                            const double xq = u53(w0, rs.next()) * Lam;
+                            int lo = 0, hi = ns - 1;
+                            while (lo < hi) {   // first j with scum[j] > xq
+                                const int mid = (lo + hi) >> 1;
+                                if (scum[mid] > xq) hi = mid;
+                                else lo = mid + 1;
+                            }
+                            acc.add(1.0, A.s_h[reg + lo], A.s_word[reg + lo], A.sp_par + reg + lo, pstride, A.npar,
+                                    L);
+                            if (REC) gz_record(A, A.s_word[reg + lo], f, r, 1.0, true);
+                        }
+                    }
+                }
             }
+            c = c1;
+            base = base_next;
         }
-        if (active) gz_store<MODE, LM, NP>(A, acc, ((int64_t)f * A.nchunks + chunk) * R + r);
     }
+    if (active) gz_store<MODE, LM, NP>(A, acc, ((int64_t)f * A.nchunks + chunk) * R + r);
 }
 
 // Records without a table (lambda above the threshold or a window larger than
@@ -1475,7 +1476,7 @@ __global__ void __launch_bounds__(GZ_BIG_THREADS, 3) k_gz_big(GapArgs A) {
     for (int tile = t0; tile < t1; tile++) nbig += A.cnt[((int64_t)f * A.ntiles + tile) * 3 + 2];
     if (nbig == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    for (int rbase = 0; rbase < R; rbase += GZ_BIG_THREADS) {
+    for (int rbase = blockIdx.z * GZ_BIG_THREADS; rbase < R; rbase += gridDim.z * GZ_BIG_THREADS) {
         const int rb = min(GZ_BIG_THREADS, R - rbase);
         const bool on = tid < rb;
         const int r = rbase + tid;
@@ -1695,14 +1696,19 @@ static size_t gz_need(int64_t B, int F, int R, int L, int npar, int tpc, int key
     return s + 512;
 }
 
-// Tiles per item that the draw wants: 8 where that leaves at least GZ_MIN_ITEMS items (5 per
-// resident workgroup; larger items mean fewer partials to write and merge), else fewer: with 8
+// Tiles per item that the draw wants: 8 where that leaves at least GZ_MIN_ITEMS workgroups (5 per
+// resident one; larger items mean fewer partials to write and merge), else fewer: with 8
 // everywhere the 61 x 51 x 41 x 20 GW-driven grid had 600 items for 768 resident workgroups, the
-// longest 17.4 ms.
+// longest 17.4 ms.  Each GZ_MAXBS realizations are a workgroup of their own: they share no tables in
+// any case, and the partials of smaller items stay below 2 x 4096 x 512 x (8 + 8 npar + 12 L) bytes
+// whatever R is.  (One workgroup for all of an item's realizations: 120,000 bins x 20, GW-driven, L = 5,
+// R = 10,000 took 66.5 ms and 3.49 GB with items of one tile, 168 ms and 1.09 GB with 4: 62 and 0.70 GB
+// so; R = 500 is one pass either way, 3.3 ms.)
 constexpr int64_t GZ_MIN_ITEMS = 4096;
-static int gz_tpc_wanted(int64_t B, int F) {
+static int gz_tpc_wanted(int64_t B, int F, int R) {
+    const int64_t passes = cdiv(R, GZ_MAXBS);
     int g = GZ_TPC_MAX;
-    while (g > 1 && cdiv(cdiv(B, GZ_TILE), g) * F < GZ_MIN_ITEMS) g >>= 1;
+    while (g > 1 && cdiv(cdiv(B, GZ_TILE), g) * F * passes < GZ_MIN_ITEMS) g >>= 1;
     return g;
 }
 
@@ -1710,7 +1716,7 @@ static int gz_tpc_wanted(int64_t B, int F) {
 // fixed scratch of hd_realize_noalloc with items of 8 tiles stays within it.
 static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
     const size_t most = gz_need(B, F, R, L, npar, GZ_TPC_MAX, 12);
-    const size_t want = gz_need(B, F, R, L, npar, gz_tpc_wanted(B, F), 12);
+    const size_t want = gz_need(B, F, R, L, npar, gz_tpc_wanted(B, F, R), 12);
     if (most > HD_NOALLOC_SCRATCH_BYTES) return std::max(most, want);
     return std::max(most, std::min(want, (size_t)HD_NOALLOC_SCRATCH_BYTES));
 }
@@ -1719,7 +1725,7 @@ static size_t gz_ws(int64_t B, int F, int R, int L, int npar) {
 // function of the sizes and mode alone, so that every entry point sums in the same order.)
 static int gz_tpc(int64_t B, int F, int R, int L, int npar, int mode) {
     const size_t have = gz_ws(B, F, R, L, npar);
-    int g = gz_tpc_wanted(B, F);
+    int g = gz_tpc_wanted(B, F, R);
     while (g < GZ_TPC_MAX && gz_need(B, F, R, L, npar, g, mode == HD_SEL_SORTED ? 4 : 12) > have) g <<= 1;
     return g;
 }
@@ -1728,11 +1734,13 @@ template <int MODE, int LM, int NP, bool REC>
 static int gz_launch_k(const GapArgs& A, dim3 grid, int bs, size_t lds, hipStream_t st) {
     {
         KTimer timer("k_gz_draw", st);
-        hipLaunchKernelGGL((k_gz_draw<MODE, LM, NP, REC>), dim3(grid.x * grid.y), dim3(bs), lds, st, A);
+        hipLaunchKernelGGL((k_gz_draw<MODE, LM, NP, REC>), dim3(grid.x * grid.y * A.px, (unsigned)cdiv(cdiv(A.R, bs), A.px)),
+                           dim3(bs), lds, st, A);
     }
     int rc = check_launch("k_gz_draw");
     if (rc) return rc;
-    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), grid, dim3(GZ_BIG_THREADS), 0, st, A);
+    const dim3 big(grid.x, grid.y, (unsigned)std::min<int64_t>(cdiv(A.R, GZ_BIG_THREADS), 65535));
+    hipLaunchKernelGGL((k_gz_big<MODE, LM, NP, REC>), big, dim3(GZ_BIG_THREADS), 0, st, A);
     return check_launch("k_gz_big");
 }
 
@@ -1833,6 +1841,11 @@ static int realize_impl(const double* number, const double* h2fdf, const int64_t
     const int64_t prep_blocks = cdiv(A.ntiles, GZ_XCDS) * GZ_XCDS * cdiv(F, GZ_PREP_FG);
     if (prep_blocks > 0x7fffffffll) return set_error(HD_ERR_SIZE, "hd_realize: too many tiles x frequencies");
     if ((int64_t)A.nchunks * F > 0x7fffffffll) return set_error(HD_ERR_SIZE, "hd_realize: too many chunks x frequencies");
+    // an item's passes run next to each other (the heaviest start first) while the launch's threads along x
+    // stay well below 2^32
+    const int64_t items = (int64_t)A.nchunks * F, passes = cdiv(R, bs);
+    A.px = (int)std::min(passes, std::max<int64_t>(1, (1 << 22) / items));
+    if (cdiv(passes, A.px) > 65535) return set_error(HD_ERR_SIZE, "hd_realize: R=%d too large", R);
     hipLaunchKernelGGL(k_gz_prep, dim3((unsigned)prep_blocks), dim3(GZ_TILE), 0, st, A);
     int rc = check_launch("k_gz_prep");
     if (rc) return rc;
