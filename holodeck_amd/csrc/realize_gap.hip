@@ -1061,10 +1061,11 @@ struct GzDraw {
     uint64_t word;
     int n, off, kt, kb;
 };
-typedef uint32_t gz_u32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t gz_u32x8 __attribute__((ext_vector_type(8), aligned(16)));
 typedef const __attribute__((address_space(4))) gz_u32x8* gz_cdraw;
 typedef const __attribute__((address_space(4))) double* gz_cpar;
 static_assert(sizeof(DRec) == 48, "a record's draw part is its first 32 bytes");
+static_assert(sizeof(DRec) % alignof(gz_u32x8) == 0, "records lie 48 bytes apart");
 __device__ __forceinline__ GzDraw gz_load_draw(const DRec* rec) {
     const gz_u32x8 w = *(gz_cdraw)rec;
     GzDraw d;
