@@ -254,6 +254,8 @@ class MLPSurrogate:
     def predict(self, X, chunk=1 << 17):
         """log10 h_c percentile spectra (M, n_out) for parameters X (M, n_in)."""
         X = np.asarray(X, dtype=float)
+        if chunk < 1:
+            raise ValueError(f"chunk={chunk}: at least one row")
         net = self._net()
         if net is not None and X.ndim == 2 and X.shape[0] > 0 and X.shape[1] == self.sizes[0]:
             # scaling to and from the training box on the device: the same double operations
