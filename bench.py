@@ -171,7 +171,7 @@ def surrogate_bench(n, judge_frac, seed=7):
     t0 = time.perf_counter()
     net.predict(X)
     t_inf = time.perf_counter() - t0
-    gemm_ms, gemm_n = _lib.timing_read("k_mlp_gemm")
+    gemm_ms, gemm_n = _lib.timing_read("k_mlp_forward")
     _lib.timing_enable(False)
     flops = 2.0 * n * sum(a * b for a, b in zip(net.sizes[:-1], net.sizes[1:]))
     sw = surrogate.SurrogateWithFallback(net, ps, nfreqs=F, nreals=int(net.meta['nreals']))

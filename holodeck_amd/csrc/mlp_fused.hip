@@ -466,7 +466,7 @@ extern "C" int hd_mlp_forward(const hd_mlp_net* net, const void* x, const double
         return set_error(HD_ERR_ARG, "hd_mlp_forward: bad arguments");
     hipStream_t st = (hipStream_t)stream;
     const FuInput in = {(const bf16*)x, raw, scale};
-    KTimer timer("k_mlp_gemm", st);
+    KTimer timer("k_mlp_forward", st);
     if (M <= FU_SMALL_ROWS) forward_launch<1>(*net, in, M, y, out, st);
     else forward_launch<4>(*net, in, M, y, out, st);
     return check_launch("k_mlp_forward");
