@@ -73,7 +73,8 @@ __device__ __forceinline__ int bessel_above(int a, double x) {
 // Low orders run the recurrence from a start that is good for any argument: the reference's upward
 // recurrence to order n + 2 multiplies the two values' last bits by (2 / e)^2 and more, which for the
 // low harmonics of nearly circular binaries is visible in g(n, e), so they keep one sequence of
-// operations for every use.  (Above ECC_LOW_ORDER the harmonics of such binaries are themselves
+// operations for every use, from sqrt(160 n) orders above n (the start of Numerical Recipes' bessj,
+// Press et al., section 6.5).  (Above ECC_LOW_ORDER the harmonics of such binaries are themselves
 // negligible, (e / 2)^(2 n).)  Bound by the chain of multiply-adds, three operations a step: the order
 // is carried as a double, the two results are taken where the first of two loops ends and, for the high
 // orders, the even orders' sum takes two of every four terms and overflow is looked for every four steps

@@ -422,7 +422,7 @@ static bool fu_ok(const hd_mlp_net* n) {
     return true;
 }
 
-// Layout of the training workspace at w (w = null: only its size); 0 where the network does not fit.
+// Layout of the training workspace at w (w = null: only its size).
 static size_t fu_layout(const hd_mlp_net* n, int M, char* w, FuBatch* B) {
     size_t s = 0;
     auto take = [&](size_t bytes) {

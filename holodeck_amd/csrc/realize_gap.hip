@@ -49,8 +49,8 @@
 //                 sparse records (cumulative lambda); the tile's cost estimate;
 //   k_gz_plan  -- one workgroup: the draw workgroups' dispatch order, (chunk,
 //                 frequency) items by decreasing estimated cost;
-//   k_gz_draw  -- per (chunk of up to 8 tiles, frequency) workgroup, one realization
-//                 per thread: tables of consecutive records are built in LDS
+//   k_gz_draw  -- per (chunk of up to 8 tiles, frequency, 512 realizations) workgroup, one
+//                 realization per thread: tables of consecutive records are built in LDS
 //                 in batches that fit (a lane per short table, a 16-lane row
 //                 per mid-size table, a wave per long one); then every
 //                 realization draws from them;
@@ -213,8 +213,9 @@ __device__ __forceinline__ double gz_pmf_acc(double lam, double k) {
 }
 
 // Estimated draw time of a tile in units of 1 ns: about 0.7 us per dense record, 1.5 ns per
-// table entry and 1.6 us per expected sparse point (a least-squares fit to the draw
-// workgroups' times at 91x81x101, F=40, R=500, R^2 0.94); the dispatch plan sorts by it.
+// table entry and 1.6 us per expected sparse point (a least-squares fit, R^2 0.94, to the draw
+// workgroups' times at 91x81x101, F=40, R=500 when the launch took 8 ms; builds and draws have both
+// become cheaper and the fit was not made again); the dispatch plan uses the order it gives.
 __device__ __forceinline__ double gz_tile_cost(int nd, int ntab, double lam_sparse) {
     return 700.0 * nd + 1.5 * ntab + 1600.0 * lam_sparse;
 }
@@ -762,7 +763,7 @@ __device__ __forceinline__ void gz_part_write(gz_lrec rec, gz_lds_u32* hi, GzPar
 }
 
 // Parts of each of nl long tables for a workgroup of GZ_WAVES waves; below GZ_SPLIT_MIN counts
-// summed over them the parts' own anchors and scans cost more than the shorter recurrence gives.
+// summed over them the parts' second barrier and scans cost more than the shorter recurrence gives.
 constexpr int GZ_WAVES = GZ_MAXBS / 64;
 #ifndef HD_GZ_SPLIT_MIN
 #define HD_GZ_SPLIT_MIN 2048
@@ -818,8 +819,8 @@ __device__ __forceinline__ void gz_build_seq(gz_lds_u32* hi, double lam, int kt,
 // lower tail (kt > kb) or j = n go to the tail walk (which takes w if the search
 // did not), else the count is kt + j.  hi[n] (the first low word) may be read by
 // the search but is not used.  (The candidate is carried as an address, so a
-// step costs one add, one compare and one select, on 4-byte words.)  Two searches
-// run interleaved (gz_draw2) so their LDS round trips overlap.
+// step costs one add, one compare and one select, on 4-byte words.)  Four searches
+// (gz_draw4) or two (gz_draw2) run interleaved so their LDS round trips overlap.
 struct GzSearch {
     const gz_lds_u32* hi;
     const gz_lds_u32* p;   // invariant: the first j with hi[j] >= x is in [p - hi, p - hi + len]
@@ -1249,11 +1250,10 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
             if (active) {
                 // dense records of the batch (one control path, so the running list needs no
                 // copies between branches), then the tile's sparse pseudo-record if it is here
-                // (records in pairs, their searches interleaved; n = 0: no table, drawn by k_gz_big)
-                // the records' fields are the same for every lane: read through the constant
-                // address space (scalar loads into SGPRs, no VALU moves); the staged LDS copy
-                // serves the builds and the rare tail walk
-                // the next pair's records are loaded before the current pair is drawn
+                // (records in fours, their searches interleaved, or in pairs where a four does not go
+                // through; n = 0: no table, drawn by k_gz_big).  The records' fields are the same for
+                // every lane: read through the constant address space (scalar loads into SGPRs, no VALU
+                // moves); the staged LDS copy serves the builds and the rare tail walk
                 const int cd = min(c1, nd);
                 const DRec* rec = A.drec + rreg;
                 {
@@ -1339,7 +1339,7 @@ __global__ void __launch_bounds__(GZ_MAXBS, 6) k_gz_draw(GapArgs A) {
 // their next attempt (attempt i of a stream is Philox block i, so a draw's state is its number and i).
 // The factors that depend on lambda alone are made once per record.  Bound by VALU issue.  (Eccentric
 // realizations, 52,111 nodes x 600 columns x 100, 8.3 million such records: 66.7 ms with a thread per
-// realization, 36.1 with the records shared by groups of waves and a lane per draw, 12.8 so; at
+// realization, 36.1 with the records shared by groups of waves and a lane per draw, 13.7 so; at
 // most 168 registers, so that the three workgroups the LDS holds fit: 26.7 with the compiler free.)
 constexpr int GZ_BIG_THREADS = 256;
 constexpr int GZ_BIG_WAVES = GZ_BIG_THREADS / 64;
@@ -1650,15 +1650,15 @@ static size_t gz_align(size_t x) { return (x + 255) & ~(size_t)255; }
 // threads beyond R only build tables (eight waves share the builds at any R).
 static int gz_block(int) { return GZ_MAXBS; }
 // LDS table capacity (8-byte slots) of every draw workgroup: table + sparse
-// axis + staged record headers + the build counter stay within 50 KB, so that
-// three workgroups fit one CU's 160 KB (allocation granularity included).
+// axis + staged record headers take 51,200 bytes, the lists, parts and counters of
+// the builds 1.7 KB more, so that three workgroups fit one CU's 160 KB.
 // Fixed, so that which bins get a table (and so every draw) does not depend
 // on the launch shape.
 #ifndef HD_GZ_CAP
 #define HD_GZ_CAP 5120
 #endif
 static int gz_cap(int) { return HD_GZ_CAP; }
-// draw workgroup LDS: table + sparse axis + staged headers (+ the build counter); three must fit a
+// draw workgroup's dynamic LDS: table + sparse axis + staged headers; three workgroups must fit a
 // 160 KB CU (with the 64 KB per-workgroup limit of the allocation), and the hook's table as well
 constexpr size_t GZ_DRAW_LDS = (size_t)(HD_GZ_CAP + GZ_TILE) * sizeof(double) + (size_t)GZ_BATCH_REC * sizeof(BRec);
 static_assert(GZ_BATCH_REC == 128, "two record ends per lane");

@@ -1117,7 +1117,7 @@ extern "C" int hd_scatter(double* dens, int M, int Q, int Z, int G, const double
     int max_lds = 0;
     if (he == hipSuccess) he = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
     if (he != hipSuccess) return set_error(HD_ERR_HIP, "hd_scatter: device query: %s", hipGetErrorString(he));
-    // the pipelined sweeps when the ring, the step tables and CT_SLOT lanes per vertex of the
+    // the pipelined sweeps when the ring, the step tables and CT_PIPE_LANES lanes per vertex of the
     // widest step fit
     const int K = ct_ring(n_levels, sweep_period);
     if (K > 0 && max_step_width > 0) {
