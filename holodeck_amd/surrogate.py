@@ -182,7 +182,7 @@ class MLPSurrogate:
             self.y_mean, self.y_std = D.to_host(mean), D.to_host(std)
         else:
             mean, std = D.to_dev(self.y_mean), D.to_dev(self.y_std)
-        X01 = torch.as_tensor(self._x01(X), dtype=torch.float32).to(D.require_device())
+        X01 = torch.as_tensor(self._x01(X), dtype=torch.float32).to(D.require_device()).contiguous()
         Yn = ((Yn - mean) / std).to(torch.float32)
         S = X.shape[0]
         gen = torch.Generator(device="cpu").manual_seed(seed)
