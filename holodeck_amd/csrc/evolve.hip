@@ -447,10 +447,11 @@ __global__ void __launch_bounds__(DBN_THREADS, 5) k_dbn_2pwl(EvoConsts K, const 
     // time past the age of the universe) it stays there, as times and rest-frame frequencies grow; the
     // margins of 1e-3 and 1e-6 cover the rounding of time_left, at most a few 1e-16 of a total time
     // that is required to be below 1e6 ages (4e-7 of time_left, and of 1 + z).  Evolutions that do not
-    // grow so (a negative normalisation, an initial separation inside the ISCO, times that are not
-    // finite) walk every step.
+    // grow so (a negative normalisation or characteristic radius, an initial separation inside the ISCO,
+    // times that are not finite) walk every step.
     const double dx_log = s_dt[0];   // the steps' spacing in log10 separation
-    const bool grows = sorted_f && norm >= 0.0 && dx_log > 1e-9 && s_tevo[nsteps] <= 1e6 * age_universe && fo[0] > 0.0;
+    const bool grows = sorted_f && norm >= 0.0 && rchar > 0.0 && dx_log > 1e-9 &&
+                       s_tevo[nsteps] <= 1e6 * age_universe && fo[0] > 0.0;
     const double f_past = 1.001 * fo[F - 1], t_past = (1.0 + 1e-6) * age_universe, t_safe = 1e-3 * age_universe;
     int step0 = 0;
     if (grows) {
