@@ -79,7 +79,10 @@ __device__ __forceinline__ int bessel_above(int a, double x) {
 // is carried as a double, the two results are taken where the first of two loops ends and, for the high
 // orders, the even orders' sum takes two of every four terms and overflow is looked for every four steps
 // (61 x 51 x 61 nodes x 40 frequencies x 100 harmonics, with the cube root below: 1.79 -> 0.40 ms).
+// TINY: x may be below 1e-12 lo.  g(n, e), with x = n e and e >= ECC_ZERO_LIMIT, does without that test
+// (1.3% of the sums' time).
 constexpr int ECC_LOW_ORDER = 6;
+template <bool TINY>
 __device__ __noinline__ void bessel_pair(int lo, double x, double& j_lo, double& j_hi) {
     if (lo < -1 || lo > ECC_MAX_ORDER || !(x > 0.0) || !(x <= ECC_MAX_ARG)) {
         j_lo = j_hi = __builtin_nan("");
@@ -104,9 +107,9 @@ __device__ __noinline__ void bessel_pair(int lo, double x, double& j_lo, double&
         }
     };
     double norm;
-    // (tiny arguments, for their order or at all: a term is 2 k / x times the one before it.  From
+    // (tiny arguments, at all or for their order: a term is 2 k / x times the one before it.  From
     // 4e-15 (a + 2) on that is below 2e15, and four steps from 1e240 stay below 2e301)
-    if (a <= ECC_LOW_ORDER || x < 1e-12 || x < 4e-15 * (double)(a + 2)) {
+    if (a <= ECC_LOW_ORDER || x < 1e-12 || (TINY && x < 4e-15 * (double)(a + 2))) {
         const double big = fmax((double)(a + 2), x);
         const int m = 2 * ((int)(big + sqrt(160.0 * big) + 10.0) / 2);
         k = (double)m;
@@ -170,7 +173,7 @@ __device__ double gw_freq_dist(int nn, double ee) {
     const double ne = nn * ee;
     const double n2 = (double)nn * nn;
     double jn_m2, jn_m1;
-    bessel_pair(nn - 2, ne, jn_m2, jn_m1);
+    bessel_pair<false>(nn - 2, ne, jn_m2, jn_m1);
     const double jn = (2 * (nn - 1) / ne) * jn_m1 - jn_m2;
     const double jn_p1 = (2 * nn / ne) * jn - jn_m1;
     const double jn_p2 = (2 * (nn + 1) / ne) * jn_p1 - jn;
@@ -409,7 +412,7 @@ __global__ void k_bessel_pair(const int* __restrict__ lo, const double* __restri
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     double a, b;
-    bessel_pair(lo[t], x[t], a, b);
+    bessel_pair<true>(lo[t], x[t], a, b);
     out[2 * t] = a;
     out[2 * t + 1] = b;
 }
